@@ -1211,6 +1211,49 @@ def test_matmul_vec4_and_scalar_loads_agree(bt):
             assert np.array_equal(bits(outs[0][h]), bits(want)), h
 
 
+# The wave tiles of k_matmul_f32.hip's rule (32 x 64, 32 x 32, 16 x 32, 16 x
+# 16), each with ragged rows and columns, a K that ends inside a chunk, and
+# rows that are whole vec4s or not.
+@pytest.mark.parametrize("transposed", [1, 0])
+@pytest.mark.parametrize("batches,m,n,k", [(32, 530, 2052, 36), (32, 530, 2050, 7), (16, 530, 1028, 68), (16, 523, 1031, 33), (8, 401, 1004, 100),
+                                           (8, 401, 1001, 65), (2, 17, 68, 132), (3, 33, 65, 129), (1, 1, 1, 1)])
+def test_matmul_tiles_bit_exact(transposed, batches, m, n, k):
+    """Every product rounded as the VALU rounds it and added in k order, as
+    the oracle: the matrix instruction's products include subnormal ones,
+    exact zeros of either sign and large ones."""
+    rng = np.random.default_rng(m * n + k)
+    a = (rng.standard_normal((batches, m, k)) * 10.0 ** rng.choice([-30, -3, 0, 3], (batches, m, k))).astype(np.float32)
+    a[rng.random(a.shape) < 0.05] = -0.0
+    b = (rng.standard_normal((1, n, k)) * 10.0 ** rng.choice([-12, -8, 0], (1, n, k))).astype(np.float32)
+    db = dev(b if transposed else b.transpose(0, 2, 1))
+    out = H.empty(batches * m * n * 4)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, batches, batches, transposed, H.F32, H.F16), p(dev(a)), p(db), p(out), None)
+    got = out.download(np.float32, (batches, m, n))
+    for z in (0, batches - 1):
+        assert np.array_equal(bits(got[z]), bits(O.matmul_float(O.T_F32, a[z], b[0], None, n, k))), z
+
+
+@pytest.mark.parametrize("heads,rows,first", [(112, 650, 131), (48, 650, 131), (16, 650, 3), (6, 200, 0), (2, 16, 0), (2, 47, 500)])
+def test_matmul_causal_tiles_bit_exact(heads, rows, first):
+    """The paired row tiles of masked scores: every score a query sees, in
+    each wave tile, and probs v with sums cut at each tile's last key."""
+    hd, keys = 36, first + rows
+    rng = np.random.default_rng(rows + first)
+    q = rng.standard_normal((heads, rows, hd)).astype(np.float32)
+    kc = rng.standard_normal((1, keys, hd)).astype(np.float32)
+    seen = np.arange(keys)[None, :] <= np.arange(rows)[:, None] + first
+    scores = H.empty(heads * rows * keys * 4)
+    H.call("vkml_matmul", H.MatmulParams(rows, keys, hd, 0, heads, heads, 1, H.F32, H.F16, 1, first), p(dev(q)), p(dev(kc)), p(scores), None)
+    got = scores.download(np.float32, (heads, rows, keys))
+    probs = rng.random((heads, rows, keys), dtype=np.float32) * seen
+    out = H.empty(heads * rows * hd * 4)
+    H.call("vkml_matmul", H.MatmulParams(rows, hd, keys, 0, heads, heads, 0, H.F32, H.F16, 1, first), p(dev(probs)), p(dev(kc)), p(out), None)
+    o = out.download(np.float32, (heads, rows, hd))
+    for h in (0, heads - 1):
+        assert np.array_equal(bits(got[h][seen]), bits(O.matmul_float(O.T_F32, q[h], kc[0], None, keys, hd)[seen])), h
+        assert np.array_equal(bits(o[h]), bits(O.matmul_float(O.T_F32, probs[h], np.ascontiguousarray(kc[0].T), None, hd, keys))), h
+
+
 @pytest.mark.parametrize("rows,first", [(130, 0), (64, 70), (200, 3)])
 def test_matmul_causal_skip_changes_nothing(rows, first):
     """The causal skip: scores on and below the diagonal (row r sees keys

@@ -1,7 +1,7 @@
 // k_ops.hip -- the decode path's small kernels and the rest of the op set:
 // quantize/dequantize, RMSNorm (+ fused activation quantize), RoPE (+ fused
 // cast and KV append), cast, row copies, permute, elementwise, embeddings,
-// argmax, softmax and a tiled f32 matmul, plus the decode-state helpers.
+// argmax and softmax, plus the decode-state helpers.
 // Where the result is integer or bit-level (codes, scales, casts, copies,
 // argmax) it is exactly the reference's; products and sums that the
 // reference writes separately are rounded separately here (plain operators
@@ -614,126 +614,6 @@ __global__ void k_embedding(vkml_embedding_params p, const void* values, const v
     }
 }
 
-// ---------------------------------------------------------------- matmul
-
-// matmul.comp's order: every output sums a[m][k] * b(k, n) in k order, a
-// product and an add at a time (matmul.comp:131-140). A 256-thread
-// workgroup computes a 64 x 64 block of c, each thread the 4 x 4 outputs at
-// rows 4 ty.., columns 4 tx..; K steps by 16 through LDS, both tiles stored
-// k-major so a thread reads its 4 rows and 4 columns as one 16-byte word
-// each. b is f32/f16/bf16, or (transposed, one batch) a quantized matrix
-// widened as gemv's weights are.
-// Four consecutive elements of a float b (f32, or f16/bf16 bits) at element e
-// (a multiple of 4, the row's base aligned), widened to f32.
-template <uint32_t BTYPE>
-__device__ __forceinline__ float4 load_b4(const void* b, uint64_t e) {
-    if constexpr (BTYPE == VKML_F32) {
-        return *reinterpret_cast<const float4*>(static_cast<const float*>(b) + e);
-    } else {
-        const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(b) + e);
-        return make_float4(half_to_float(w.x & 0xFFFFu, BTYPE), half_to_float(w.x >> 16, BTYPE), half_to_float(w.y & 0xFFFFu, BTYPE),
-                           half_to_float(w.y >> 16, BTYPE));
-    }
-}
-
-// VEC (float b, rows of a and of b whole vec4s, aligned): each thread loads
-// a's and b's tile elements as one vec4 each instead of four scalars.
-template <bool BT, uint32_t BTYPE, bool VEC = false>
-__global__ void __launch_bounds__(256) k_matmul(vkml_matmul_params p, const float* a, const void* b, const void* bs, float* c) {
-    // Rows of 68: stores that run along k hit 16 different banks.
-    __shared__ __align__(16) float ta[16][68], tb[16][68];
-    const uint32_t tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
-    const uint32_t row0 = blockIdx.y * 64, col0 = blockIdx.x * 64, z = blockIdx.z;
-    // Under a causal mask the tile's last row sees keys up to row0 + 63 +
-    // offset: scores past it are never read, and a's entries past it are 0.
-    const uint64_t last_key = static_cast<uint64_t>(row0) + 63 + p.causal_offset;
-    if (BT && p.causal && col0 > last_key) return;
-    const uint32_t k_end = (!BT && p.causal) ? static_cast<uint32_t>(min<uint64_t>(p.k, last_key + 1)) : p.k;
-    const float* az = a + static_cast<uint64_t>(z) * p.m * p.k;
-    const uint64_t b_off = static_cast<uint64_t>(z / p.b_group) * p.b_stride;
-    const auto b_at = [&](uint32_t n, uint32_t k) -> float {
-        if constexpr (BTYPE >= VKML_Q8_0) {
-            return weight_value(BTYPE, p.scale_type, b, bs, p.k, n, k);
-        } else {
-            const uint64_t e = b_off + (BT ? static_cast<uint64_t>(n) * p.k + k : static_cast<uint64_t>(k) * p.n + n);
-            return load_src(b, e, BTYPE);
-        }
-    };
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-    for (uint32_t k0 = 0; k0 < k_end; k0 += 16) {
-        // Out-of-range elements are zeros, which add nothing.
-        if constexpr (VEC) {
-            {  // a: row tid / 4, k0 + 4 (tid % 4) ..
-                const uint32_t r = tid / 4, kq = tid % 4, row = row0 + r, k = k0 + 4 * kq;
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (row < p.m && k < p.k) v = *reinterpret_cast<const float4*>(az + static_cast<uint64_t>(row) * p.k + k);
-                ta[4 * kq][r] = v.x;
-                ta[4 * kq + 1][r] = v.y;
-                ta[4 * kq + 2][r] = v.z;
-                ta[4 * kq + 3][r] = v.w;
-            }
-            if constexpr (BT) {  // b [n, k]: column tid / 4, k0 + 4 (tid % 4) ..
-                const uint32_t col = tid / 4, kq = tid % 4, n = col0 + col, kg = k0 + 4 * kq;
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (n < p.n && kg < p.k) v = load_b4<BTYPE>(b, b_off + static_cast<uint64_t>(n) * p.k + kg);
-                tb[4 * kq][col] = v.x;
-                tb[4 * kq + 1][col] = v.y;
-                tb[4 * kq + 2][col] = v.z;
-                tb[4 * kq + 3][col] = v.w;
-            } else {  // b [k, n]: k0 + tid / 16, columns 4 (tid % 16) ..
-                const uint32_t kb = tid / 16, cq = tid % 16, n = col0 + 4 * cq, kg = k0 + kb;
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (n < p.n && kg < p.k) v = load_b4<BTYPE>(b, b_off + static_cast<uint64_t>(kg) * p.n + n);
-                *reinterpret_cast<float4*>(&tb[kb][4 * cq]) = v;
-            }
-        } else {
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const uint32_t e = tid + 256 * u;
-            const uint32_t r = e / 16, kk = e % 16, row = row0 + r, k = k0 + kk;
-            ta[kk][r] = (row < p.m && k < p.k) ? az[static_cast<uint64_t>(row) * p.k + k] : 0.0f;
-            uint32_t col, kb;
-            if (BT) {  // b is [n, k]: run along k
-                col = e / 16;
-                kb = e % 16;
-            } else {  // b is [k, n]: run along n
-                kb = e / 64;
-                col = e % 64;
-            }
-            const uint32_t n = col0 + col, kg = k0 + kb;
-            tb[kb][col] = (n < p.n && kg < p.k) ? b_at(n, kg) : 0.0f;
-        }
-        }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t kk = 0; kk < 16; ++kk) {
-            const float4 av = *reinterpret_cast<const float4*>(&ta[kk][4 * ty]);
-            const float4 bv = *reinterpret_cast<const float4*>(&tb[kk][4 * tx]);
-            const float ar[4] = {av.x, av.y, av.z, av.w}, br[4] = {bv.x, bv.y, bv.z, bv.w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += ar[i] * br[j];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t row = row0 + 4 * ty + i;
-        if (row >= p.m) continue;
-        float* cr = c + (static_cast<uint64_t>(z) * p.m + row) * p.n;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t col = col0 + 4 * tx + j;
-            if (col < p.n) cr[col] = acc[i][j];
-        }
-    }
-}
-
 }  // namespace
 
 extern "C" {
@@ -993,59 +873,5 @@ int vkml_step_finish(uint32_t vocab, const float* logits, vkml_decode_state* sta
     hipLaunchKernelGGL(k_step_finish, dim3(1), dim3(1024), 0, S(), vocab, logits, state, log, cap);
     return vkml::abi::check_launch("step_finish");
 }
-
-int vkml_matmul(const vkml_matmul_params* p, const float* a, const void* b, float* c, const void* b_scales) {
-    VKML_REQUIRE_INIT();
-    VKML_CHECK_ARG(p, "matmul: null params");
-    VKML_CHECK_ARG(p->b_type <= VKML_Q4_K, "matmul: unknown b type " + std::to_string(p->b_type));
-    VKML_CHECK_ARG(p->b_group >= 1 && p->batches >= 1, "matmul: bad batching");
-    const bool quant = p->b_type >= VKML_Q8_0;
-    VKML_CHECK_ARG(!p->causal || !quant, "matmul: the causal skip is for attention's products, not weights");
-    if (quant) {
-        VKML_CHECK_ARG(p->b_transposed && p->batches == 1, "matmul: quantized b must be one transposed [n, k] matrix");
-        const uint32_t unit = p->b_type == VKML_Q4_K ? 256 : 32;
-        VKML_CHECK_ARG(p->k % unit == 0, "matmul: k = " + std::to_string(p->k) + " is not whole blocks of " + std::to_string(unit));
-        VKML_CHECK_ARG(p->scale_type == VKML_F16 || (p->scale_type == VKML_F32 && p->b_type != VKML_Q4_K),
-                       "matmul: bad scale type");
-        VKML_CHECK_ARG(b_scales, "matmul: quantized b needs scales");
-    }
-    if (p->m == 0 || p->n == 0) return VKML_OK;
-    VKML_CHECK_ARG(a && b && c, "matmul: null buffer");
-    VKML_CHECK_ARG((p->m + 63) / 64 <= 65535 && p->batches <= 65535, "matmul: too many rows or batches");
-    const dim3 grid((p->n + 63) / 64, (p->m + 63) / 64, p->batches);
-    ProfileScope prof("matmul");
-    const bool t = p->b_transposed != 0;
-    // Whole, aligned vec4s along k in a's rows (and b's when transposed),
-    // along n in b's rows otherwise.
-    const bool vec = p->b_type <= VKML_BF16 && p->k % 4 == 0 && (t || p->n % 4 == 0) && p->b_stride % 4 == 0 &&
-                     reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(b) % (p->b_type == VKML_F32 ? 16 : 8) == 0;
-    if (vec) {
-        const auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, S(), *p, a, b, b_scales, c); };
-        if (p->b_type == VKML_F32) t ? launch(k_matmul<true, VKML_F32, true>) : launch(k_matmul<false, VKML_F32, true>);
-        else if (p->b_type == VKML_F16) t ? launch(k_matmul<true, VKML_F16, true>) : launch(k_matmul<false, VKML_F16, true>);
-        else t ? launch(k_matmul<true, VKML_BF16, true>) : launch(k_matmul<false, VKML_BF16, true>);
-        return vkml::abi::check_launch("matmul");
-    }
-    switch (p->b_type) {
-        case VKML_F32:
-            if (t) hipLaunchKernelGGL((k_matmul<true, VKML_F32>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            else hipLaunchKernelGGL((k_matmul<false, VKML_F32>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            break;
-        case VKML_F16:
-            if (t) hipLaunchKernelGGL((k_matmul<true, VKML_F16>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            else hipLaunchKernelGGL((k_matmul<false, VKML_F16>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            break;
-        case VKML_BF16:
-            if (t) hipLaunchKernelGGL((k_matmul<true, VKML_BF16>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            else hipLaunchKernelGGL((k_matmul<false, VKML_BF16>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c);
-            break;
-        case VKML_Q8_0: hipLaunchKernelGGL((k_matmul<true, VKML_Q8_0>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c); break;
-        case VKML_Q4_0: hipLaunchKernelGGL((k_matmul<true, VKML_Q4_0>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c); break;
-        case VKML_Q4_1: hipLaunchKernelGGL((k_matmul<true, VKML_Q4_1>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c); break;
-        default: hipLaunchKernelGGL((k_matmul<true, VKML_Q4_K>), grid, dim3(256), 0, S(), *p, a, b, b_scales, c); break;
-    }
-    return vkml::abi::check_launch("matmul");
-}
-
 
 }  // extern "C"
