@@ -1211,6 +1211,25 @@ def test_matmul_vec4_and_scalar_loads_agree(bt):
             assert np.array_equal(bits(outs[0][h]), bits(want)), h
 
 
+@pytest.mark.parametrize("bt", [H.F32, H.F16, H.BF16])
+@pytest.mark.parametrize("n,k", [(1, 4), (33, 128), (70, 132), (9, 256), (17, 260), (8, 1024), (23, 1028), (40, 4104), (5, 66)])
+def test_gemv_float_loads_bit_exact(bt, n, k):
+    """vkml_gemv with a float b, 1 to 8 rows of a: a group of four a load for
+    rows of whole aligned groups (short rows, and longer ones in chunks of
+    1024, whole or not), the general kernel for other k's and for an a that
+    starts off alignment: all the oracle's order, bit for bit."""
+    rng = np.random.default_rng(n * k + bt)
+    dv, _, ot, ob, _ = _float_b(bt, n, k, rng)
+    for m in range(1, 9):
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        want = O.gemv_float(ot, a, ob, None, n, k)
+        shifted = dev(np.concatenate([np.zeros(1, np.float32), a.ravel()]))
+        for ptr in (p(dev(a)), C.c_void_p(p(shifted).value + 4)):
+            out = H.empty(m * n * 4)
+            H.call("vkml_gemv", H.GemvParams(m, n, k, bt, H.F16, 0, 1, 1), ptr, p(dv), p(out), None)
+            assert np.array_equal(bits(out.download(np.float32, (m, n))), bits(want)), m
+
+
 # The wave tiles of k_matmul_f32.hip's rule (32 x 64, 32 x 32, 16 x 32, 16 x
 # 16), each with ragged rows and columns, a K that ends inside a chunk, and
 # rows that are whole vec4s or not.

@@ -6,6 +6,7 @@
 // are used when 8 would leave SIMDs idle (the N = 4096 projections of a 7B
 // model: 4096 rows x 16 lanes is one wave per SIMD).
 #include <algorithm>
+#include <type_traits>
 
 #include "device.hpp"
 #include "gemv.hpp"
@@ -281,6 +282,179 @@ __global__ void __launch_bounds__(256) k_gemv_float(const float* a, uint32_t m, 
     }
 }
 
+// The same order for a float b whose rows are whole, aligned groups of four
+// (k % 4 == 0): a lane loads a group with one 8- or 16-byte load, U steps of
+// R rows at once, the next batch's loads in flight while this one is summed.
+// For rows of one or two steps (scores of 32 heads of 128 against 4000 keys:
+// two queries 20 -> 11 us, eight 30 -> 23.5).
+template <int BT>
+using Group4 = std::conditional_t<BT == VKML_F32, uint4, uint2>;
+
+template <int BT>
+__device__ __forceinline__ float4 widen4(Group4<BT> w) {
+    if constexpr (BT == VKML_F32) return make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
+    else return make_float4(half_to_float(w.x & 0xFFFFu, BT), half_to_float(w.x >> 16, BT), half_to_float(w.y & 0xFFFFu, BT),
+                            half_to_float(w.y >> 16, BT));
+}
+
+template <int BT, int M, int R, int U>
+__global__ void __launch_bounds__(256) k_gemv_float4(const float* a, uint32_t m, const void* b, float* out, uint32_t n, uint32_t k,
+                                                     uint32_t b_group, uint64_t b_stride) {
+#pragma clang fp contract(off)
+    constexpr uint32_t kSize = BT == VKML_F32 ? 4 : 2;
+    const uint32_t z = blockIdx.y, lane = threadIdx.x % 32, groups = k / 4;
+    a += static_cast<uint64_t>(z) * m * k;
+    out += static_cast<uint64_t>(z) * m * n;
+    const uint8_t* bz = static_cast<const uint8_t*>(b) + static_cast<uint64_t>(z / b_group) * b_stride * kSize;
+    const uint32_t row0 = (blockIdx.x * 8 + threadIdx.x / 32) * R;
+    const Group4<BT>* br[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) br[r] = reinterpret_cast<const Group4<BT>*>(bz + static_cast<uint64_t>(min(row0 + r, n - 1)) * k * kSize);
+    const float4* ar[M];  // (rows past m repeat the last one, and are not stored)
+#pragma unroll
+    for (int q = 0; q < M; ++q) ar[q] = reinterpret_cast<const float4*>(a + static_cast<uint64_t>(min(static_cast<uint32_t>(q), m - 1)) * k);
+    struct Batch {
+        Group4<BT> w[U][R];
+        float4 x[U][M];
+    };
+    const auto load = [&](uint32_t s, Batch& d) {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t i = min(32 * (s + u) + lane, groups - 1);
+#pragma unroll
+            for (int r = 0; r < R; ++r) d.w[u][r] = ldg(br[r] + i);
+#pragma unroll
+            for (int q = 0; q < M; ++q) d.x[u][q] = ldg(ar[q] + i);
+        }
+    };
+    float acc[M][R];
+#pragma unroll
+    for (int q = 0; q < M; ++q)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[q][r] = 0.0f;
+    const auto step = [&](uint32_t u, const Batch& d) {
+        float4 w[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r] = widen4<BT>(d.w[u][r]);
+#pragma unroll
+        for (int q = 0; q < M; ++q) {
+            const float4 x = d.x[u][q];
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[q][r] += x.x * w[r].x + x.y * w[r].y + x.z * w[r].z + x.w * w[r].w;
+        }
+    };
+    const uint32_t steps = (groups + 31) / 32;
+    Batch cur, next;
+    load(0, cur);
+    for (uint32_t s = 0; s < steps; s += U) {
+        if (s + U < steps) load(s + U, next);
+        if (32 * (s + U) <= groups) {
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) step(u, cur);
+        } else {
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u)
+                if (32 * (s + u) + lane < groups) step(u, cur);
+        }
+        cur = next;
+    }
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        if (q >= static_cast<int>(m)) break;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float v = tree_to_first<32>(acc[q][r]);  // strides 16 .. 1 toward the row's lane 0
+            if (lane == 0 && row0 + r < n) out[static_cast<uint64_t>(q) * n + row0 + r] = v;
+        }
+    }
+}
+
+// The same for longer rows: a's groups, which every row of b needs, are
+// staged in LDS, eight steps (1024 values of each row of a) at a time, the
+// next chunk's loads of a and of b in flight meanwhile. Bound by reading b
+// (one row of b a half wave, us against the kernel above it, which loads an
+// element at a time and waits for each group): bf16 14336 x 4096, one row of
+// a 39.8 -> 23.4 (5.0 TB/s), five 77.3 -> 34.5, eight 107 -> 45; 4096 x
+// 14336 84.1 -> 24.2, 198 -> 46.6, 281 -> 56; two rows of b a half wave lose
+// at n = 4096 (51.5 against 37 at four rows of a). From six rows of a on, the
+// products and sums, two VALU operations each, weigh as much as b.
+template <int BT, int M>
+__global__ void __launch_bounds__(256) k_gemv_float4_rows(const float* a, uint32_t m, const void* b, float* out, uint32_t n, uint32_t k,
+                                                          uint32_t b_group, uint64_t b_stride) {
+#pragma clang fp contract(off)
+    constexpr uint32_t kSize = BT == VKML_F32 ? 4 : 2;
+    constexpr uint32_t U = 8;
+    __shared__ float4 xs[M][32 * U];
+    const uint32_t z = blockIdx.y, t = threadIdx.x, lane = t % 32, groups = k / 4;
+    a += static_cast<uint64_t>(z) * m * k;
+    out += static_cast<uint64_t>(z) * m * n;
+    const uint8_t* bz = static_cast<const uint8_t*>(b) + static_cast<uint64_t>(z / b_group) * b_stride * kSize;
+    const uint32_t row = blockIdx.x * 8 + t / 32;
+    const Group4<BT>* br = reinterpret_cast<const Group4<BT>*>(bz + static_cast<uint64_t>(min(row, n - 1)) * k * kSize);
+    const float4* a4 = reinterpret_cast<const float4*>(a);
+    float4 xa[M];  // group t of the chunk, of every row of a (rows past m repeat the last one, and are not stored)
+    Group4<BT> cur[U], next[U];
+    const auto load = [&](uint32_t s, Group4<BT> (&w)[U]) {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) w[u] = ldg(br + min(32 * (s + u) + lane, groups - 1));
+#pragma unroll
+        for (int q = 0; q < M; ++q) xa[q] = ldg(a4 + static_cast<uint64_t>(min(static_cast<uint32_t>(q), m - 1)) * groups + min(32 * s + t, groups - 1));
+    };
+    float acc[M];
+#pragma unroll
+    for (int q = 0; q < M; ++q) acc[q] = 0.0f;
+    const uint32_t steps = (groups + 31) / 32;
+    load(0, cur);
+    for (uint32_t s = 0; s < steps; s += U) {
+        __syncthreads();  // the last chunk's readers are done
+#pragma unroll
+        for (int q = 0; q < M; ++q) xs[q][t] = xa[q];
+        __syncthreads();
+        if (s + U < steps) load(s + U, next);
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (32 * (s + u) + lane < groups) {
+                const float4 w = widen4<BT>(cur[u]);
+#pragma unroll
+                for (int q = 0; q < M; ++q) {
+                    const float4 x = xs[q][32 * u + lane];
+                    acc[q] += x.x * w.x + x.y * w.y + x.z * w.z + x.w * w.w;
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) cur[u] = next[u];
+    }
+#pragma unroll
+    for (int q = 0; q < M; ++q) {
+        if (q >= static_cast<int>(m)) break;
+        const float v = tree_to_first<32>(acc[q]);  // strides 16 .. 1 toward the row's lane 0
+        if (lane == 0 && row < n) out[static_cast<uint64_t>(q) * n + row] = v;
+    }
+}
+
+template <int BT>
+void launch_float4(const vkml_gemv_params& p, const float* a, const void* b, float* out, uint32_t batches, uint32_t group) {
+    const auto go = [&](auto kernel, uint32_t rows) {
+        hipLaunchKernelGGL(kernel, dim3((p.n + 8 * rows - 1) / (8 * rows), batches), dim3(256), 0, vkml::abi::stream(), a, p.m, b, out, p.n, p.k,
+                           group, static_cast<uint64_t>(p.b_stride));
+    };
+    if (p.k <= 256) {
+        // One or two steps a row (attention's scores of up to 8 queries):
+        // several rows a lane keep as many loads in flight, and a is read
+        // from the caches.
+        if (p.m == 1) go(k_gemv_float4<BT, 1, 4, 2>, 4);
+        else if (p.m == 2) go(k_gemv_float4<BT, 2, 4, 2>, 4);
+        else if (p.m <= 4) go(k_gemv_float4<BT, 4, 2, 1>, 2);
+        else if (p.m <= 6) go(k_gemv_float4<BT, 6, 2, 1>, 2);
+        else go(k_gemv_float4<BT, 8, 2, 1>, 2);
+    } else if (p.m == 1) go(k_gemv_float4_rows<BT, 1>, 1);
+    else if (p.m == 2) go(k_gemv_float4_rows<BT, 2>, 1);
+    else if (p.m <= 4) go(k_gemv_float4_rows<BT, 4>, 1);
+    else if (p.m <= 6) go(k_gemv_float4_rows<BT, 6>, 1);
+    else go(k_gemv_float4_rows<BT, 8>, 1);
+}
+
 }  // namespace
 
 extern "C" {
@@ -415,6 +589,15 @@ int vkml_gemv(const vkml_gemv_params* p, const float* a, const void* b, float* o
     VKML_CHECK_ARG(a && b && out, "gemv: null buffer");
     const dim3 grid((p->n + 7) / 8, batches);
     vkml::abi::ProfileScope prof("gemv");
+    // Whole, aligned groups of four in a's rows and a float b's.
+    const uint32_t unit = p->b_type == VKML_F32 ? 16 : 8;
+    if (p->b_type <= VKML_BF16 && p->k % 4 == 0 && p->k > 0 && p->b_stride % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
+        reinterpret_cast<uintptr_t>(b) % unit == 0) {
+        if (p->b_type == VKML_F32) launch_float4<VKML_F32>(*p, a, b, out, batches, group);
+        else if (p->b_type == VKML_F16) launch_float4<VKML_F16>(*p, a, b, out, batches, group);
+        else launch_float4<VKML_BF16>(*p, a, b, out, batches, group);
+        return vkml::abi::check_launch("gemv");
+    }
     hipStream_t s = vkml::abi::stream();
     const uint64_t bst = p->b_stride;
 #define VKML_GEMV_LAUNCH(T) \
