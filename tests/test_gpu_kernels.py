@@ -1211,6 +1211,24 @@ def test_matmul_vec4_and_scalar_loads_agree(bt):
             assert np.array_equal(bits(outs[0][h]), bits(want)), h
 
 
+@pytest.mark.parametrize("fmt", [H.Q8_0, H.Q4_0, H.Q4_1, H.Q4_K])
+@pytest.mark.parametrize("n,k", [(1, 256), (9, 512), (37, 1792), (16, 2048), (50, 2304), (25, 4096), (21, 96)])
+def test_gemv_dot_two_to_eight_rows_bit_exact(fmt, n, k):
+    """The rows kernel's chunks of four rounds (2048 values): whole, a part of
+    one, several and a remainder, for every number of rows, in the oracle's
+    order bit for bit."""
+    if fmt == H.Q4_K and k % 256:
+        k = 256 * (k // 256 + 1)
+    v, s, quant, words, scales = weights(fmt, n, k, n + k)
+    a, aw, asc = activation(k, k, 8)
+    da, ds = dev(aw), dev(asc)
+    want = O.gemv_dot(quant, aw, asc, 8, words, scales, n, k)
+    for m in range(2, 9):
+        out = H.empty(m * n * 4)
+        H.call("vkml_gemv_dot", H.GemvDotParams(m, n, k, fmt, H.F16), p(da), p(v), p(out), p(s), p(ds))
+        assert np.array_equal(bits(out.download(np.float32, (m, n))), bits(np.asarray(want)[:m])), m
+
+
 @pytest.mark.parametrize("bt", [H.F32, H.F16, H.BF16])
 @pytest.mark.parametrize("n,k", [(1, 4), (33, 128), (70, 132), (9, 256), (17, 260), (8, 1024), (23, 1028), (40, 4104), (5, 66)])
 def test_gemv_float_loads_bit_exact(bt, n, k):

@@ -163,47 +163,104 @@ int check_dot_params(const vkml_gemv_dot_params* p, const char* what, bool any_k
 // ---------------------------------------------------------------- several rows
 
 // gemv_dot for 2 .. 8 activation rows in one launch (gemv_dot.comp handles
-// its M rows in one dispatch): each round of a weight row is loaded once and
-// applied to every activation row, each row with its own accumulators in
-// the single-row kernel's order (the same lanes, terms and halving tree).
-// LPR lanes an output row (32 for q8_0 and q4_K, 16 for q4_0 and q4_1);
-// the activation codes are read from memory (the workgroup's rows share
-// them in L1), the next round's weights in flight during this one.
-template <int FMT, bool F16S, int LPR, bool FULL>
+// its M rows in one dispatch): each round of a weight row is loaded and
+// unpacked once and applied to every activation row, each row with its own
+// accumulators in the single-row kernel's order (the same lanes, terms and
+// halving tree). LPR lanes an output row. K runs in chunks of four rounds:
+// the workgroup stages the chunk's codes, code sums and scales of every
+// activation row in LDS, and the next chunk's weights and activations are in
+// flight meanwhile. At two rows bound by reading the weights; each further
+// row adds ten VALU operations and 24 bytes from LDS a half-block and lane,
+// which bound it from four on. Against reading the activations from the
+// caches and summing their codes a lane (us; two, five and eight rows):
+// q4_K 14336 x 4096 17.6, 24.5, 32.3 -> 11.4, 17.7, 20.7; 4096 x 14336 23.1,
+// 28.9, 35.0 -> 11.5, 17.7, 21.0; q8_0 4096 x 14336 22.5, 26.4, 31.1 -> 12.2,
+// 16.5, 19.2; q4_0 14336 x 4096 12.7, 21.9, 30.1 -> 10.0, 16.3, 19.5. (Two
+// weight rows a lane sharing the LDS reads: within 5% either way.)
+template <int FMT, bool F16S, int LPR, bool FULL, int M>
 __global__ void __launch_bounds__(256) k_gemv_dot_rows(GemvArgs g, uint32_t m) {
     constexpr int NS = Plan<FMT, LPR>::NS;
-    constexpr uint32_t kRows = 256 / LPR;
+    constexpr uint32_t kRows = 256 / LPR, CR = 4, H = 32 * CR, NL = M * H / 256;
+    __shared__ uint4 s_codes[M][H];
+    __shared__ float2 s_ss[M][H];
     const uint32_t t = thread_index(), l = t % LPR, grp = t / LPR;
     const uint32_t out_row = blockIdx.x * kRows + grp, row = min(out_row, g.n - 1);
     const uint32_t K = g.k, halves = K / 16, rounds = (halves + 31) / 32;
     const Q4kField jf = q4k_field((l % 16) / 2);
-    float acc[8][NS];
+    // Rows past m repeat the last one and are not stored; half-blocks past K
+    // repeat its last one and are skipped.
+    uint4 codes[NL];
+    float scale[NL];
+    const auto load_act = [&](uint32_t r0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+        for (uint32_t u = 0; u < NL; ++u) {
+            const uint32_t e = t + 256 * u, i = min(e / H, m - 1), hb = min(32 * r0 + e % H, halves - 1);
+            codes[u] = ldg(g.a_values + static_cast<uint64_t>(i) * halves + hb);
+            scale[u] = ldg(g.a_scales + static_cast<uint64_t>(i) * (K / 32) + hb / 2);
+        }
+    };
+    RoundW<FMT, LPR> w[CR], next[CR];
+    const auto load_weights = [&](uint32_t r0, RoundW<FMT, LPR> (&d)[CR]) {
+#pragma unroll
+        for (uint32_t u = 0; u < CR; ++u) load_round<FMT, F16S, LPR>(g.b_values, g.b_scales, K, row, min(r0 + u, rounds - 1), l, d[u]);
+    };
+    float acc[M][NS];
+#pragma unroll
+    for (int i = 0; i < M; ++i)
 #pragma unroll
         for (int e = 0; e < NS; ++e) acc[i][e] = 0.0f;
-    RoundW<FMT, LPR> w;
-    load_round<FMT, F16S, LPR>(g.b_values, g.b_scales, K, row, 0, l, w);
-    for (uint32_t r = 0; r < rounds; ++r) {
-        RoundW<FMT, LPR> next;
-        load_round<FMT, F16S, LPR>(g.b_values, g.b_scales, K, row, min(r + 1, rounds - 1), l, next);
+    load_act(0);
+    load_weights(0, w);
+    for (uint32_t r0 = 0; r0 < rounds; r0 += CR) {
+        __syncthreads();  // the last chunk's readers are done
 #pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            if (i >= m) break;
-            RoundA<FMT, LPR> x;
+        for (uint32_t u = 0; u < NL; ++u) {
+            const uint32_t e = t + 256 * u;
+            s_codes[e / H][e % H] = codes[u];
+            s_ss[e / H][e % H] = make_float2(static_cast<float>(byte_sum(codes[u])), scale[u]);
+        }
+        __syncthreads();
+        if (r0 + CR < rounds) {
+            load_act(r0 + CR);
+            load_weights(r0 + CR, next);
+        }
+        // Two activation rows at a time, the next two's LDS reads issued before
+        // this two's arithmetic (left to itself the compiler waits for each
+        // read where it issues it).
+        RoundA<FMT, LPR> x[2][2];
+        const auto fetch = [&](uint32_t u, uint32_t i, RoundA<FMT, LPR>& d) {
 #pragma unroll
             for (int e = 0; e < NS; ++e) {
-                const uint32_t hb = min(32 * r + acc_index<FMT, LPR>(l, e), halves - 1);
-                x.a[e] = ldg(g.a_values + static_cast<uint64_t>(i) * halves + hb);
-                x.ss[e] = make_float2(static_cast<float>(byte_sum(x.a[e])), ldg(g.a_scales + static_cast<uint64_t>(i) * (K / 32) + hb / 2));
+                const uint32_t hb = 32 * u + acc_index<FMT, LPR>(l, e);
+                d.a[e] = s_codes[i][hb];
+                d.ss[e] = s_ss[i][hb];
             }
-            round_terms<FMT, F16S, LPR, FULL>(w, x, r, l, K, jf, acc[i]);
+        };
+        fetch(0, 0, x[0][0]);
+        fetch(0, 1, x[0][1]);
+#pragma unroll
+        for (uint32_t u = 0; u < CR; ++u) {
+            if (r0 + u >= rounds) break;
+#pragma unroll
+            for (uint32_t i = 0; i < M; i += 2) {
+                const uint32_t p = (u * (M / 2) + i / 2) % 2;
+                if (i + 2 < M || u + 1 < CR) {
+                    const uint32_t nu = i + 2 < M ? u : u + 1, ni = i + 2 < M ? i + 2 : 0;
+                    fetch(nu, ni, x[1 - p][0]);
+                    fetch(nu, ni + 1, x[1 - p][1]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                round_terms<FMT, F16S, LPR, FULL>(w[u], x[p][0], r0 + u, l, K, jf, acc[i]);
+                round_terms<FMT, F16S, LPR, FULL>(w[u], x[p][1], r0 + u, l, K, jf, acc[i + 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        w = next;
+#pragma unroll
+        for (uint32_t u = 0; u < CR; ++u) w[u] = next[u];
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 8; ++i) {
-        if (i >= m) break;
+    for (int i = 0; i < M; ++i) {
+        if (i >= static_cast<int>(m)) break;
         const float v = row_tree<FMT, LPR>(acc[i]);
         // + residual (one activation row): add(x, y), llama.cpp:374,386
         if (l == 0 && out_row < g.n) g.out[static_cast<uint64_t>(i) * g.n + out_row] = g.residual ? ldg(g.residual + out_row) + v : v;
@@ -212,11 +269,18 @@ __global__ void __launch_bounds__(256) k_gemv_dot_rows(GemvArgs g, uint32_t m) {
 
 template <int FMT, bool F16S>
 int launch_rows(const GemvArgs& g, uint32_t m) {
+    // 32 lanes a row where the format has them (16 lanes, half the waves and
+    // twice the accumulators a lane: 24.5 against 18.1 us at 14336 x 4096,
+    // q4_K, five rows).
     constexpr int LPR = FMT == VKML_Q8_0 || FMT == VKML_Q4_K ? 32 : 16;
     const dim3 grid((g.n + 256 / LPR - 1) / (256 / LPR));
     vkml::abi::ProfileScope prof("gemv_dot");
-    if (g.k % 512 == 0) hipLaunchKernelGGL((k_gemv_dot_rows<FMT, F16S, LPR, true>), grid, dim3(256), 0, vkml::abi::stream(), g, m);
-    else hipLaunchKernelGGL((k_gemv_dot_rows<FMT, F16S, LPR, false>), grid, dim3(256), 0, vkml::abi::stream(), g, m);
+    const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, vkml::abi::stream(), g, m); };
+    const bool full = g.k % 512 == 0;
+    if (m <= 2) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 2>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 2>);
+    else if (m <= 4) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 4>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 4>);
+    else if (m <= 6) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 6>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 6>);
+    else full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 8>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 8>);
     return vkml::abi::check_launch("gemv_dot");
 }
 
