@@ -279,6 +279,26 @@ def test_matmul_dot_bit_exact(fmt, f16, m, n, k):
         assert np.all(np.abs(got - exact) <= bound)
 
 
+@pytest.mark.parametrize("fmt,f16", [(H.Q8_0, True), (H.Q8_0, False), (H.Q4_0, True), (H.Q4_1, True), (H.Q4_1, False), (H.Q4_K, True)])
+@pytest.mark.parametrize("m,n,k", [(9, 70, 96), (33, 65, 288), (17, 1000, 2336), (150, 2500, 544), (119, 8200, 544), (139, 8200, 32),
+                                   (530, 3872, 800), (2050, 8200, 288)])
+def test_matmul_dot_tiles_bit_exact(fmt, f16, m, n, k):
+    # The four tiles of launch()'s rule (16 x 64 in the first four, 16 x 128
+    # and 32 x 128 with 1028 and 1285 or more waves of 32 x 32, 64 x 128),
+    # ragged both ways, with a K that ends inside a chunk of 8 blocks and of
+    # one, two and several chunks.
+    if fmt == H.Q4_K:
+        k = 256 * (k // 256 + 1)
+    v, s, quant, words, scales = weights(fmt, n, k, m + n, f16_scales=f16)
+    a, aw, asc = activation(k, m, m)
+    out = H.empty(m * n * 4)
+    H.call("vkml_matmul_dot", H.GemvDotParams(m, n, k, fmt, H.F16 if f16 else H.F32), p(dev(aw)), p(v), p(out), p(s), p(dev(asc)))
+    got = out.download(np.float32, (m, n))
+    rows = np.unique(np.concatenate([np.arange(min(m, 20)), np.arange(max(m - 20, 0), m), np.arange(0, m, 61)]))
+    aw, asc = np.ascontiguousarray(aw.reshape(m, -1)[rows]), np.ascontiguousarray(asc.reshape(m, -1)[rows])
+    assert np.array_equal(bits(got[rows]), bits(O.matmul_dot(quant, aw, asc, len(rows), words, scales, n, k)))
+
+
 @pytest.mark.parametrize("fmt", [H.Q8_0, H.Q4_K])
 def test_gemv_dot_add_and_swiglu(fmt):
     n, k = 1024, 4096

@@ -20,22 +20,24 @@
 // Lane l of a wave holds, for a 16 x 16 instruction, a's row l % 16 and b's
 // column l % 16 at the block's values 8 (l / 16) .. 8 (l / 16) + 7 (one
 // 8-byte operand each), and gets the results for rows 4 (l / 16) .. + 3 of
-// column l % 16. K runs in chunks of 8 blocks; for each chunk the
-// workgroup stages every row's (scale, code sum) and every column's (scale,
-// offset) per block in LDS, and the scaling reads four rows' values as one
-// 16-byte word. The large-product kernel also stages the chunk's operands
-// in LDS, copied with 16-byte loads a chunk ahead in registers (2x the
-// kernel that loads each block's 8-byte operands from memory, whose waves
-// spent twice their issue time waiting for them); the small tiles load
-// operands straight from memory (L2 serves the reuse across workgroups).
-// The scaling costs 4 VALU operations per output and block (the offset
-// formats' six folded into four, as block_term says), and it bounds the
-// kernel: a SIMD issues a wave64 f32 VALU instruction about every 4
-// cycles (measured 33.7 T lane-operations a second for fma, 36.8 T for mul,
-// 38.7 T for add over the GPU), so 4 operations per output and block cap
-// the kernel near 9 T outputs x blocks a second, about 580 TOP/s of the
-// int8 products (11.6% of the int8 peak); the matrix instructions are idle
-// most of the time.
+// column l % 16. K runs in chunks of 8 blocks, staged in LDS with 16-byte
+// loads a chunk ahead in registers: the operands, every row's
+// (scale, code sum) and every column's (scale, offset) per block; the
+// scaling reads four rows' values as one 16-byte word.
+//
+// What bounds it. The scaling costs 4 operations per output and block (the
+// offset formats' six folded into four, as kSumBiasBits says), which issue at
+// 1.0 (mul, add) to 1.25 ns (fma) a wave64 instruction on a SIMD with two
+// waves or more ready, and the matrix instructions, 7 ns each, hide little of
+// it: 5.7 ns for a lane's output and block, 740 TOP/s, when nothing waits.
+// The large products reach 480 TOP/s, the 512-row ones 360 to 440. One
+// operation in four is an outer product of a row tile's and a column tile's
+// values, which the matrix unit forms for sixteen outputs a lane at once
+// (add_tiles); with the others run sixteen at a time that took 512 x 14336 x
+// 4096 (q4_K) from 156 to 148 us, 512 x 4096 x 14336 181 -> 166, 1000 x 8192
+// x 3072 (q4_1) 143 -> 128. The 16 x 64 tiles replace kernels that loaded
+// operands from memory block by block: 131 x 2048 x 8192 (q8_0) 130 -> 52 us,
+// 37 x 4096 x 14336 145 -> 66, 9 x 4096 x 4096 34 -> 20.
 #include <algorithm>
 
 #include "../../include/vkml_hip.h"
@@ -48,6 +50,7 @@ namespace {
 
 constexpr uint32_t kT = 256;      // four waves
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 struct MatmulDotArgs {
     const uint8_t* a;     // [M, K] activation codes
@@ -72,38 +75,6 @@ __device__ __forceinline__ float f16_at(const void* p, uint64_t i) { return f16_
 // nibbles of a word minus 8 (matmul_dot.comp:71-73).
 __device__ __forceinline__ uint32_t q4_signed(uint32_t word, uint32_t shift) {
     return (((word >> shift) & 0x0F0F0F0Fu) + 0x78787878u) ^ 0x80808080u;
-}
-
-// Column n's operand for block blk: its 8 codes at values 8 g .. 8 g + 7 of
-// the block, as int8 (q4: codes 0 .. 15, or minus 8 for q4_0).
-template <int FMT>
-__device__ __forceinline__ long b_codes(const MatmulDotArgs& p, uint32_t n, uint32_t blk, uint32_t g) {
-    uint32_t lo, hi;
-    if constexpr (FMT == VKML_Q8_0) {
-        const uint2 w = ldg(reinterpret_cast<const uint2*>(p.b + static_cast<uint64_t>(n) * p.k + blk * 32 + 8 * g));
-        lo = w.x;
-        hi = w.y;
-    } else if constexpr (FMT == VKML_Q4_K) {
-        // sub-block j = blk % 8 of super-block blk / 8: low (j even) or high
-        // nibbles of bytes 32 (j / 2) .. of its 128
-        const uint32_t j = blk % 8, sb = blk / 8;
-        const uint2 w = ldg(reinterpret_cast<const uint2*>(p.b + static_cast<uint64_t>(n) * (p.k / 2) + sb * 128 + 32 * (j / 2) + 8 * g));
-        const uint32_t sh = 4 * (j % 2);
-        lo = (w.x >> sh) & 0x0F0F0F0Fu;
-        hi = (w.y >> sh) & 0x0F0F0F0Fu;
-    } else {
-        // QuantizedMatrix q4 words: word w' of the block holds values 8 w' .. 8 w' + 7,
-        // low nibbles the first four, high the last four
-        const uint32_t q = ldg(reinterpret_cast<const uint32_t*>(p.b + static_cast<uint64_t>(n) * (p.k / 2) + blk * 16 + 4 * g));
-        if constexpr (FMT == VKML_Q4_0) {
-            lo = q4_signed(q, 0);
-            hi = q4_signed(q, 4);
-        } else {
-            lo = q & 0x0F0F0F0Fu;
-            hi = (q >> 4) & 0x0F0F0F0Fu;
-        }
-    }
-    return static_cast<long>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
 // Column n's scale and offset for block blk (q8_0 / q4_0: offset unused).
@@ -167,6 +138,46 @@ __device__ __forceinline__ v4i sum_start() {
     return v4i{b, b, b, b};
 }
 
+// A 16 RT x 64 CT tile with its operands staged in LDS: per 8-block chunk
+// the workgroup copies the chunk's A rows (16 RT x 256 bytes) and B columns
+// (64 CT x 128 bytes, 256 for q8_0) with 16-byte loads, a chunk ahead in
+// registers, and the matrix instructions read their operands from LDS. Each staging thread's A bytes are whole blocks of one row (two at RT =
+// 4, one below; at RT = 1 half the threads stage A), so it also sums their
+// codes.
+template <int FMT, bool F16S, int RT, int CT>
+struct StagedChunk {
+    static constexpr bool kOffset = FMT == VKML_Q4_1 || FMT == VKML_Q4_K;
+    static constexpr uint32_t TM = 16 * RT, TN = 64 * CT;     // the tile
+    static constexpr bool kMask = RT * CT != 8;               // blocks past K are computed, as zeros (the largest tile stops at K)
+    static constexpr uint32_t kABlocks = RT >= 2 ? RT / 2 : 1;  // a staging thread's A blocks (of one row)
+    static constexpr uint32_t kAThreads = TM * kChunk / kABlocks;  // threads that stage A
+    static constexpr uint32_t kBBytes = FMT == VKML_Q8_0 ? 256 : 128;  // a column's bytes a chunk
+    static constexpr uint32_t kAStride = 272, kBStride = kBBytes + 16;  // padded rows: no bank conflicts
+    static constexpr uint32_t kBLoads = kBBytes * TN / 16 / kT;         // 16-byte B loads a thread
+    static constexpr uint32_t kSThreads = 2 * TN < kT ? 2 * TN : kT;     // threads that stage columns' scales, four blocks of
+    static constexpr uint32_t kSCols = 2 * TN / kSThreads;              // this many columns each
+    uint4 a[2 * kABlocks];
+    uint4 b[kBLoads];
+    float sa[kABlocks];
+    uint4 header[kSCols];
+    float s[kSCols][4], o[kSCols][4];
+};
+
+template <int FMT, bool F16S, int RT, int CT>
+struct StagedLds {
+    using S = StagedChunk<FMT, F16S, RT, CT>;
+    alignas(16) uint8_t a[S::TM * S::kAStride];
+    alignas(16) uint8_t b[S::TN * S::kBStride];
+    alignas(16) float sa[kChunk][S::TM];
+    alignas(16) float asum[kChunk][S::kOffset ? S::TM : 4];
+    float sb[kChunk][S::TN];
+    float ob[kChunk][S::kOffset ? S::TN : 1];
+};
+
+// Keeps the VALU instructions before it before those after it; the others
+// (LDS reads, matrix instructions, scalar ones) may cross.
+__device__ __forceinline__ void valu_stage() { __builtin_amdgcn_sched_barrier(0x3FC); }
+
 // One output's contribution of one block, sa (sum sb + asum ob) or
 // sum (sa sb) (matmul_dot.comp:155-160), from the matrix instruction's
 // result d (biased where the scaling folds; nsb = -1.5 * 2^23 * sb).
@@ -183,156 +194,121 @@ __device__ __forceinline__ float block_term(int32_t d, float sa, float asum, flo
     }
 }
 
-// One kernel per per-wave tile: RT row tiles of 16 by CT column tiles of
-// 16; a workgroup's four waves take 4 CT column tiles side by side, so its
-// tile is 16 RT x 64 CT.
+// A block's operands of the scaling: the wave's rows' scales and code sums
+// (rows 4 g .. + 3 of each row tile), its columns' scales and offsets.
+template <int RT, int CT>
+struct BlockStats {
+    float4 sa[RT], asum[RT];
+    float sb[CT], nsb[CT], ob[CT];
+};
+
+// The results of G blocks' RT x CT tiles (d) into the accumulators, block by
+// block in each: one operation of all sixteen terms a lane, then the next, so
+// that no operation waits for the one before it. (Left to itself the compiler
+// forms each term's four dependent operations in a row.)
+template <int FMT, bool F16S, int RT, int CT, int G>
+__device__ __forceinline__ void add_tiles(const v4i (&d)[G][RT][CT], const BlockStats<RT, CT> (&st)[G], const StagedLds<FMT, F16S, RT, CT>& l,
+                                          uint32_t block, uint32_t wave, uint32_t lane, float (&acc)[RT][CT][4]) {
+#pragma clang fp contract(off)
+    static_assert(RT * CT * G == 4);
+    // What a row and a column give together, the code sums times the offsets
+    // or the two scales, are outer products of a row tile's and a column
+    // tile's sixteen: one v_mfma_f32_16x16x1_4b_f32 forms them for four tiles
+    // from one value a lane of each, each rounded as the VALU rounds it
+    // (fma(asum, ob, x) on the scaled sums; sa * sb on zeros, where a -0 comes
+    // out +0, which no accumulator can tell).
+    constexpr bool kScales = FMT == VKML_Q8_0 || FMT == VKML_Q4_0;
+    if constexpr (kFoldScaling<FMT, F16S> || kScales) {
+        const uint32_t blk = lane / 16, li = lane % 16, q = blk / (RT * CT), cl = 16 * CT * wave + 16 * (blk / RT % CT) + li;
+        float row, col;
+        if constexpr (kScales) {
+            row = l.sa[block + q][16 * (blk % RT) + li];
+            col = l.sb[block + q][cl];
+        } else {
+            row = l.asum[block + q][16 * (blk % RT) + li];
+            col = l.ob[block + q][cl];
+        }
+        v16f t;
+        valu_stage();
+        if constexpr (kScales) {
+            const v16f u = __builtin_amdgcn_mfma_f32_16x16x1f32(row, col, v16f{}, 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t[j] = static_cast<float>(d[j / (4 * RT * CT)][j / 4 % RT][j / (4 * RT) % CT][j % 4]);
+            valu_stage();
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t[j] = t[j] * u[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int b = j / (4 * RT * CT), r = j / 4 % RT, c = j / (4 * RT) % CT;
+                const int sum = d[b][r][c][j % 4];  // (bit_cast of a vector's element itself takes element 0)
+                t[j] = __builtin_fmaf(__builtin_bit_cast(float, sum), st[b].sb[c], st[b].nsb[c]);
+            }
+            t = __builtin_amdgcn_mfma_f32_16x16x1f32(row, col, t, 0, 0, 0);
+            valu_stage();
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int b = j / (4 * RT * CT), r = j / 4 % RT, i = j % 4;
+                const float4 s4 = st[b].sa[r];
+                t[j] = (i == 0 ? s4.x : i == 1 ? s4.y : i == 2 ? s4.z : s4.w) * t[j];
+            }
+        }
+        valu_stage();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j / 4 % RT][j / (4 * RT) % CT][j % 4] += t[j];
+        valu_stage();
+    } else {
+        // q4_1 with f32 scales: the reference's operations.
+#pragma unroll
+        for (int b = 0; b < G; ++b)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const float sa[4] = {st[b].sa[r].x, st[b].sa[r].y, st[b].sa[r].z, st[b].sa[r].w};
+                const float asum[4] = {st[b].asum[r].x, st[b].asum[r].y, st[b].asum[r].z, st[b].asum[r].w};
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[r][c][i] += block_term<FMT, F16S>(d[b][r][c][i], sa[i], asum[i], st[b].sb[c], st[b].nsb[c], st[b].ob[c]);
+            }
+    }
+}
+
+// The same for the 64 x 32 wave tile, one block: a row tile's terms as the
+// compiler orders them (its chains overlap those of the next row tile's, and
+// sixteen at a time needed registers that cost a wave: 4096 x 14336 x 4096
+// 1079 against 1010 us).
 template <int FMT, bool F16S, int RT, int CT>
-__global__ void __launch_bounds__(kT) k_matmul_dot(MatmulDotArgs p) {
+__device__ __forceinline__ void add_large(const v4i (&d)[RT][CT], const StagedLds<FMT, F16S, RT, CT>& l, uint32_t block, uint32_t wave,
+                                          uint32_t lane, float (&acc)[RT][CT][4]) {
 #pragma clang fp contract(off)
     constexpr bool kOffset = FMT == VKML_Q4_1 || FMT == VKML_Q4_K;
-    constexpr uint32_t TM = 16 * RT, TN = 64 * CT;
-    // Per chunk, double-buffered: rows' scales and code sums, columns'
-    // scales and offsets, [block of the chunk][row or column].
-    __shared__ __align__(16) float s_sa[2][kChunk][TM];
-    __shared__ __align__(16) float s_asum[2][kChunk][kOffset ? TM : 4];
-    __shared__ float s_sb[2][kChunk][TN];
-    __shared__ float s_ob[2][kChunk][kOffset ? TN : 1];
-    const uint32_t t = thread_index(), lane = t % kWave, wave = t / kWave;
     const uint32_t g = lane / 16, li = lane % 16;
-    const uint32_t row0 = blockIdx.y * TM, col0 = blockIdx.x * TN;
-    const uint32_t blocks = p.k / 32;
-    const uint8_t* arow[RT];
+    float sb[CT], nsb[CT], ob[CT];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) arow[r] = p.a + static_cast<uint64_t>(min(row0 + 16 * r + li, p.m - 1)) * p.k + 8 * g;
-    uint32_t bcol[CT];
+    for (int c = 0; c < CT; ++c) {
+        sb[c] = l.sb[block][16 * CT * wave + 16 * c + li];
+        nsb[c] = -kSumBias * sb[c];
+        ob[c] = 0.0f;
+        if constexpr (kOffset) ob[c] = l.ob[block][16 * CT * wave + 16 * c + li];
+    }
 #pragma unroll
-    for (int c = 0; c < CT; ++c) bcol[c] = min(col0 + 16 * CT * wave + 16 * c + li, p.n - 1);
-    float acc[RT][CT][4];
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
+    for (int r = 0; r < RT; ++r) {
+        const float4 sa4 = *reinterpret_cast<const float4*>(&l.sa[block][16 * r + 4 * g]);
+        float4 as4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if constexpr (kOffset) as4 = *reinterpret_cast<const float4*>(&l.asum[block][16 * r + 4 * g]);
+        const float sa[4] = {sa4.x, sa4.y, sa4.z, sa4.w}, asum[4] = {as4.x, as4.y, as4.z, as4.w};
 #pragma unroll
         for (int c = 0; c < CT; ++c)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[r][c][i] = 0.0f;
-
-    for (uint32_t c0 = 0, buf = 0; c0 < blocks; c0 += kChunk, buf ^= 1) {
-        // Stage the chunk's statistics: TM rows x 8 blocks, and TN columns x
-        // 8 blocks (a column's four blocks a thread).
-#pragma unroll
-        for (uint32_t e = t; e < TM * kChunk; e += kT) {
-            const uint32_t r = e % TM, b = e / TM, blk = c0 + b;
-            if (blk < blocks) {
-                const uint32_t row = min(row0 + r, p.m - 1);
-                s_sa[buf][b][r] = ldg(p.a_scales + static_cast<uint64_t>(row) * blocks + blk);
-                if constexpr (kOffset) {
-                    const uint4* codes = reinterpret_cast<const uint4*>(p.a + static_cast<uint64_t>(row) * p.k + blk * 32);
-                    s_asum[buf][b][r] = static_cast<float>(byte_sum(ldg(codes)) + byte_sum(ldg(codes + 1)));
-                }
-            }
-        }
-#pragma unroll
-        for (uint32_t e = t; e < TN * 2; e += kT) {
-            const uint32_t cl = e / 2, b0 = 4 * (e % 2), col = min(col0 + cl, p.n - 1);
-            if constexpr (FMT == VKML_Q4_K) {
-                const uint4 h = ldg(reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(p.b_scales) +
-                                                                   (static_cast<uint64_t>(col) * (p.k / 256) + c0 / 8) * 16));
-#pragma unroll
-                for (uint32_t b = 0; b < 4; ++b) q4k_block_scale(h, b0 + b, s_sb[buf][b0 + b][cl], s_ob[buf][b0 + b][cl]);
-            } else {
-#pragma unroll
-                for (uint32_t b = 0; b < 4; ++b) {
-                    if (c0 + b0 + b < blocks) {
-                        float s, o;
-                        b_block_scale<FMT, F16S>(p, col, c0 + b0 + b, s, o);
-                        s_sb[buf][b0 + b][cl] = s;
-                        if constexpr (kOffset) s_ob[buf][b0 + b][cl] = o;
-                    }
-                }
-            }
-        }
-        __syncthreads();  // the chunk's statistics are staged (the other buffer's readers finished a chunk ago)
-#pragma unroll
-        for (uint32_t b = 0; b < kChunk; ++b) {
-            const uint32_t blk = c0 + b;
-            if (blk >= blocks) break;
-            long av[RT], bv[CT];
-#pragma unroll
-            for (int r = 0; r < RT; ++r) av[r] = static_cast<long>(__builtin_bit_cast(uint64_t, ldg(reinterpret_cast<const uint2*>(arow[r] + blk * 32))));
-#pragma unroll
-            for (int c = 0; c < CT; ++c) bv[c] = b_codes<FMT>(p, bcol[c], blk, g);
-            float sb[CT], nsb[CT], ob[CT];
-#pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                sb[c] = s_sb[buf][b][16 * CT * wave + 16 * c + li];
-                nsb[c] = -kSumBias * sb[c];
-                ob[c] = 0.0f;
-                if constexpr (kOffset) ob[c] = s_ob[buf][b][16 * CT * wave + 16 * c + li];
-            }
-#pragma unroll
-            for (int r = 0; r < RT; ++r) {
-                const float4 sa4 = *reinterpret_cast<const float4*>(&s_sa[buf][b][16 * r + 4 * g]);
-                float4 as4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if constexpr (kOffset) as4 = *reinterpret_cast<const float4*>(&s_asum[buf][b][16 * r + 4 * g]);
-                const float sa[4] = {sa4.x, sa4.y, sa4.z, sa4.w}, asum[4] = {as4.x, as4.y, as4.z, as4.w};
-#pragma unroll
-                for (int c = 0; c < CT; ++c) {
-                    const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[r], bv[c], sum_start<FMT, F16S>(), 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[r][c][i] += block_term<FMT, F16S>(d[i], sa[i], asum[i], sb[c], nsb[c], ob[c]);
-                }
-            }
-        }
+            for (int i = 0; i < 4; ++i) acc[r][c][i] += block_term<FMT, F16S>(d[r][c][i], sa[i], asum[i], sb[c], nsb[c], ob[c]);
     }
-#pragma unroll
-    for (int r = 0; r < RT; ++r)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            const uint32_t col = col0 + 16 * CT * wave + 16 * c + li;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = row0 + 16 * r + 4 * g + i;
-                if (row < p.m && col < p.n) store_out(p, row, col, acc[r][c][i]);
-            }
-        }
 }
 
-// The 16 RT x 128 tile with its operands staged in LDS: per 8-block chunk
-// the workgroup copies the chunk's A rows (16 RT x 256 bytes) and B columns
-// (128 x 128 bytes, 256 for q8_0) with 16-byte loads, a chunk ahead in
-// registers, and the matrix instructions read their operands from LDS. Each
-// staging thread's A bytes are whole blocks of one row (two at RT = 4, one
-// below; at RT = 1 half the threads stage A), so it also sums their codes.
-template <int FMT, bool F16S, int RT>
-struct StagedChunk {
-    static constexpr bool kOffset = FMT == VKML_Q4_1 || FMT == VKML_Q4_K;
-    static constexpr uint32_t TM = 16 * RT;                   // rows of the tile
-    static constexpr uint32_t kABlocks = RT >= 2 ? RT / 2 : 1;  // a staging thread's A blocks (of one row)
-    static constexpr uint32_t kAThreads = TM * kChunk / kABlocks;  // threads that stage A
-    static constexpr uint32_t kBBytes = FMT == VKML_Q8_0 ? 256 : 128;  // a column's bytes a chunk
-    static constexpr uint32_t kAStride = 272, kBStride = kBBytes + 16;  // padded rows: no bank conflicts
-    static constexpr uint32_t kBLoads = kBBytes * 128 / 16 / kT;        // 16-byte B loads a thread
-    uint4 a[2 * kABlocks];
-    uint4 b[kBLoads];
-    float sa[kABlocks];
-    uint4 header;
-    float s[4], o[4];
-};
-
-template <int FMT, bool F16S, int RT>
-struct StagedLds {
-    static constexpr bool kOffset = FMT == VKML_Q4_1 || FMT == VKML_Q4_K;
-    alignas(16) uint8_t a[16 * RT * StagedChunk<FMT, F16S, RT>::kAStride];
-    alignas(16) uint8_t b[128 * StagedChunk<FMT, F16S, RT>::kBStride];
-    alignas(16) float sa[kChunk][16 * RT];
-    alignas(16) float asum[kChunk][kOffset ? 16 * RT : 4];
-    float sb[kChunk][128];
-    float ob[kChunk][kOffset ? 128 : 1];
-};
-
-template <int FMT, bool F16S, int RT>
+template <int FMT, bool F16S, int RT, int CT>
 __device__ __forceinline__ void staged_load(const MatmulDotArgs& p, uint32_t t, uint32_t c0, uint32_t row0, uint32_t col0,
-                                            StagedChunk<FMT, F16S, RT>& r) {
-    using S = StagedChunk<FMT, F16S, RT>;
+                                            StagedChunk<FMT, F16S, RT, CT>& r) {
+    using S = StagedChunk<FMT, F16S, RT, CT>;
     constexpr uint32_t AB = S::kABlocks, kPerRow = kChunk / AB;  // threads a row
     const uint32_t blocks = p.k / 32;
     if (S::kAThreads == kT || t < S::kAThreads) {
@@ -364,21 +340,24 @@ __device__ __forceinline__ void staged_load(const MatmulDotArgs& p, uint32_t t, 
         }
         r.b[u] = ldg(reinterpret_cast<const uint4*>(src));
     }
-    {
-        const uint32_t col = min(col0 + t / 2, p.n - 1), b0 = 4 * (t % 2);
-        if constexpr (FMT == VKML_Q4_K) {
-            r.header = ldg(reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(p.b_scales) +
-                                                          (static_cast<uint64_t>(col) * (p.k / 256) + c0 / 8) * 16));
-        } else {
+    if (S::kSThreads == kT || t < S::kSThreads) {
 #pragma unroll
-            for (uint32_t b = 0; b < 4; ++b) b_block_scale<FMT, F16S>(p, col, min(c0 + b0 + b, blocks - 1), r.s[b], r.o[b]);
+        for (uint32_t u = 0; u < S::kSCols; ++u) {
+            const uint32_t col = min(col0 + t / 2 + kT / 2 * u, p.n - 1), b0 = 4 * (t % 2);
+            if constexpr (FMT == VKML_Q4_K) {
+                r.header[u] = ldg(reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(p.b_scales) +
+                                                                 (static_cast<uint64_t>(col) * (p.k / 256) + c0 / 8) * 16));
+            } else {
+#pragma unroll
+                for (uint32_t b = 0; b < 4; ++b) b_block_scale<FMT, F16S>(p, col, min(c0 + b0 + b, blocks - 1), r.s[u][b], r.o[u][b]);
+            }
         }
     }
 }
 
-template <int FMT, bool F16S, int RT>
-__device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT>& r, uint32_t t, StagedLds<FMT, F16S, RT>& l) {
-    using S = StagedChunk<FMT, F16S, RT>;
+template <int FMT, bool F16S, int RT, int CT>
+__device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT, CT>& r, uint32_t t, uint32_t left, StagedLds<FMT, F16S, RT, CT>& l) {
+    using S = StagedChunk<FMT, F16S, RT, CT>;
     constexpr bool kOffset = S::kOffset;
     constexpr uint32_t AB = S::kABlocks, kPerRow = kChunk / AB;
     if (S::kAThreads == kT || t < S::kAThreads) {
@@ -389,8 +368,12 @@ __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT>& r
 #pragma unroll
         for (uint32_t h = 0; h < AB; ++h) {
             const uint32_t b = AB * (t % kPerRow) + h;
-            l.sa[b][row] = r.sa[h];
-            if constexpr (kOffset) l.asum[b][row] = static_cast<float>(byte_sum(r.a[2 * h]) + byte_sum(r.a[2 * h + 1]));
+            // Blocks past K (the last chunk of a K of other than whole chunks)
+            // re-read its last one with zero scales, offsets and code sums:
+            // their terms are zeros, which change no accumulator (none is ever
+            // -0).
+            l.sa[b][row] = !S::kMask || b < left ? r.sa[h] : 0.0f;
+            if constexpr (kOffset) l.asum[b][row] = !S::kMask || b < left ? static_cast<float>(byte_sum(r.a[2 * h]) + byte_sum(r.a[2 * h + 1])) : 0.0f;
         }
     }
 #pragma unroll
@@ -398,20 +381,25 @@ __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT>& r
         const uint32_t e = t + kT * u, cl = e / (S::kBBytes / 16), piece = e % (S::kBBytes / 16);
         *reinterpret_cast<uint4*>(l.b + cl * S::kBStride + 16 * piece) = r.b[u];
     }
-    const uint32_t cl = t / 2, b0 = 4 * (t % 2);
+    if (S::kSThreads == kT || t < S::kSThreads) {
 #pragma unroll
-    for (uint32_t b = 0; b < 4; ++b) {
-        float sv = r.s[b], ov = r.o[b];
-        if constexpr (FMT == VKML_Q4_K) q4k_block_scale(r.header, b0 + b, sv, ov);
-        l.sb[b0 + b][cl] = sv;
-        if constexpr (kOffset) l.ob[b0 + b][cl] = ov;
+        for (uint32_t u = 0; u < S::kSCols; ++u) {
+            const uint32_t cl = t / 2 + kT / 2 * u, b0 = 4 * (t % 2);
+#pragma unroll
+            for (uint32_t b = 0; b < 4; ++b) {
+                float sv = r.s[u][b], ov = r.o[u][b];
+                if constexpr (FMT == VKML_Q4_K) q4k_block_scale(r.header[u], b0 + b, sv, ov);
+                l.sb[b0 + b][cl] = !S::kMask || b0 + b < left ? sv : 0.0f;
+                if constexpr (kOffset) l.ob[b0 + b][cl] = !S::kMask || b0 + b < left ? ov : 0.0f;
+            }
+        }
     }
 }
 
 // Column cl's operand for block b of the staged chunk (as b_codes).
-template <int FMT, bool F16S, int RT>
-__device__ __forceinline__ long staged_b(const StagedLds<FMT, F16S, RT>& l, uint32_t cl, uint32_t b, uint32_t g) {
-    using S = StagedChunk<FMT, F16S, RT>;
+template <int FMT, bool F16S, int RT, int CT>
+__device__ __forceinline__ long staged_b(const StagedLds<FMT, F16S, RT, CT>& l, uint32_t cl, uint32_t b, uint32_t g) {
+    using S = StagedChunk<FMT, F16S, RT, CT>;
     const uint8_t* col = l.b + cl * S::kBStride;
     uint32_t lo, hi;
     if constexpr (FMT == VKML_Q8_0) {
@@ -436,77 +424,82 @@ __device__ __forceinline__ long staged_b(const StagedLds<FMT, F16S, RT>& l, uint
     return static_cast<long>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-template <int FMT, bool F16S, int RT>
-__global__ void __launch_bounds__(kT) k_matmul_dot_staged(MatmulDotArgs p) {
-#pragma clang fp contract(off)
-    using S = StagedChunk<FMT, F16S, RT>;
+template <int FMT, bool F16S, int RT, int CT>
+__global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulDotArgs p) {
+    using S = StagedChunk<FMT, F16S, RT, CT>;
     constexpr bool kOffset = S::kOffset;
-    __shared__ StagedLds<FMT, F16S, RT> l;
+    constexpr int G = RT * CT >= 4 ? 1 : 4 / (RT * CT);  // blocks whose scaling runs together
+    __shared__ StagedLds<FMT, F16S, RT, CT> l;
     const uint32_t t = thread_index(), lane = t % kWave, wave = t / kWave;
     const uint32_t g = lane / 16, li = lane % 16;
-    const uint32_t row0 = blockIdx.y * S::TM, col0 = blockIdx.x * 128;
+    const uint32_t row0 = blockIdx.y * S::TM, col0 = blockIdx.x * S::TN;
     const uint32_t blocks = p.k / 32;
-    float acc[RT][2][4];
+    float acc[RT][CT][4];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int c = 0; c < CT; ++c)
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[r][c][i] = 0.0f;
-    // A block's matrix instructions (RT x 2 of them) into d.
-    const auto sums = [&](uint32_t b, v4i (&d)[RT][2]) {
-        long av[RT], bv[2];
+    // A block's matrix instructions (RT x CT of them) into d.
+    const auto sums = [&](uint32_t b, v4i (&d)[RT][CT]) {
+        long av[RT], bv[CT];
 #pragma unroll
         for (int r = 0; r < RT; ++r) av[r] = *reinterpret_cast<const long*>(l.a + (16 * r + li) * S::kAStride + b * 32 + 8 * g);
 #pragma unroll
-        for (int c = 0; c < 2; ++c) bv[c] = staged_b<FMT, F16S, RT>(l, 32 * wave + 16 * c + li, b, g);
+        for (int c = 0; c < CT; ++c) bv[c] = staged_b<FMT, F16S, RT, CT>(l, 16 * CT * wave + 16 * c + li, b, g);
 #pragma unroll
         for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int c = 0; c < 2; ++c) d[r][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[r], bv[c], sum_start<FMT, F16S>(), 0, 0, 0);
+            for (int c = 0; c < CT; ++c) d[r][c] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[r], bv[c], sum_start<FMT, F16S>(), 0, 0, 0);
     };
-    // A block's scaling of d into the accumulators, in the reference's order.
-    const auto scale = [&](uint32_t b, const v4i (&d)[RT][2]) {
-        float sb[2], nsb[2], ob[2];
+    const auto stats = [&](uint32_t b, BlockStats<RT, CT>& st) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            sb[c] = l.sb[b][32 * wave + 16 * c + li];
-            nsb[c] = -kSumBias * sb[c];
-            ob[c] = 0.0f;
-            if constexpr (kOffset) ob[c] = l.ob[b][32 * wave + 16 * c + li];
+        for (int c = 0; c < CT; ++c) {
+            const uint32_t cl = 16 * CT * wave + 16 * c + li;
+            st.sb[c] = l.sb[b][cl];
+            st.nsb[c] = -kSumBias * st.sb[c];
+            st.ob[c] = 0.0f;
+            if constexpr (kOffset) st.ob[c] = l.ob[b][cl];
         }
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-            const float4 sa4 = *reinterpret_cast<const float4*>(&l.sa[b][16 * r + 4 * g]);
-            float4 as4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if constexpr (kOffset) as4 = *reinterpret_cast<const float4*>(&l.asum[b][16 * r + 4 * g]);
-            const float sa[4] = {sa4.x, sa4.y, sa4.z, sa4.w}, asum[4] = {as4.x, as4.y, as4.z, as4.w};
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[r][c][i] += block_term<FMT, F16S>(d[r][c][i], sa[i], asum[i], sb[c], nsb[c], ob[c]);
+            st.sa[r] = *reinterpret_cast<const float4*>(&l.sa[b][16 * r + 4 * g]);
+            st.asum[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if constexpr (kOffset) st.asum[r] = *reinterpret_cast<const float4*>(&l.asum[b][16 * r + 4 * g]);
         }
     };
-    StagedChunk<FMT, F16S, RT> next;
-    staged_load<FMT, F16S, RT>(p, t, 0, row0, col0, next);
+    StagedChunk<FMT, F16S, RT, CT> next;
+    staged_load<FMT, F16S, RT, CT>(p, t, 0, row0, col0, next);
     for (uint32_t c0 = 0; c0 < blocks; c0 += kChunk) {
         __syncthreads();  // the last chunk's readers are done
-        staged_store<FMT, F16S, RT>(next, t, l);
+        staged_store<FMT, F16S, RT, CT>(next, t, blocks - c0, l);
         __syncthreads();
-        if (c0 + kChunk < blocks) staged_load<FMT, F16S, RT>(p, t, c0 + kChunk, row0, col0, next);  // in flight meanwhile
+        if (c0 + kChunk < blocks) staged_load<FMT, F16S, RT, CT>(p, t, c0 + kChunk, row0, col0, next);  // in flight meanwhile
 #pragma unroll
-        for (uint32_t b = 0; b < kChunk; ++b) {
-            if (c0 + b >= blocks) break;
-            v4i d[RT][2];
-            sums(b, d);
-            scale(b, d);
+        for (uint32_t b = 0; b < kChunk; b += G) {
+            if constexpr (RT * CT == 8) {
+                if (c0 + b >= blocks) break;  // (keeps the next block's reads, and their registers, out of this one)
+                v4i d[RT][CT];
+                sums(b, d);
+                add_large<FMT, F16S, RT, CT>(d, l, b, wave, lane, acc);
+            } else {
+                v4i d[G][RT][CT];
+                BlockStats<RT, CT> st[G];
+#pragma unroll
+                for (int q = 0; q < G; ++q) {
+                    sums(b + q, d[q]);
+                    stats(b + q, st[q]);
+                }
+                add_tiles<FMT, F16S, RT, CT, G>(d, st, l, b, wave, lane, acc);
+            }
         }
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const uint32_t col = col0 + 32 * wave + 16 * c + li;
+        for (int c = 0; c < CT; ++c) {
+            const uint32_t col = col0 + 16 * CT * wave + 16 * c + li;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t row = row0 + 16 * r + 4 * g + i;
@@ -516,41 +509,28 @@ __global__ void __launch_bounds__(kT) k_matmul_dot_staged(MatmulDotArgs p) {
 }
 
 template <int FMT, bool F16S, int RT, int CT>
-void launch_tiles(const MatmulDotArgs& p) {
+void launch_tile(const MatmulDotArgs& p) {
     const dim3 grid((p.n + 64 * CT - 1) / (64 * CT), (p.m + 16 * RT - 1) / (16 * RT));
     hipLaunchKernelGGL((k_matmul_dot<FMT, F16S, RT, CT>), grid, dim3(kT), 0, vkml::abi::stream(), p);
 }
 
-// The 64 x 128 tile with its operands staged in LDS (2x the direct-load
-// kernel at large prompts) wherever it gives every CU about four
-// workgroups; below that the 32 x 128 staged tile, wherever it gives the
-// SIMDs two waves each; below that the 16 x 128 staged tile, wherever the
-// 32-row one would give them half a wave; below that, the largest
-// direct-load tile that still gives them about two waves each. (Measured:
-// the staged tiles win from 512 of their waves on; a 512-token cfg5
-// prompt's projections take 19.1 ms with 32 x 128 tiles against 23.3 ms
-// with 64 x 128, a 4096-token prompt's 116-124 ms either way, the 64 x 128
-// tile ahead in most runs; cfg3's 512-token q|k|v, o and down, one to one
-// and a half 32-row waves a SIMD, take 25.8, 20.6 and 74.0 us with 16-row
-// tiles against 29.9, 24.4 and 89.0 us; at 128 rows x 14336 columns the
-// 32 x 32 direct tile beats 64 x 32 with half the waves and 32 x 16 with
-// twice as many.)
+// Tiles of 64 x 128, 32 x 128, 16 x 128 and 16 x 64 outputs, the larger while
+// the SIMDs still get waves enough. Measured (us; those four): q4_K 4096 x
+// 14336 x 4096 999, 1054, -, -; 4096 x 4096 x 14336 1003, 1049, -, -; 512 x
+// 14336 x 4096 169, 148, 179, 231; 512 x 4096 x 14336 245, 166, 183, 236; 300
+// x 8192 x 2048 47, 37, 36, 45; 300 x 3072 x 2048 37, 23, 18, 21; 300 x 2048 x
+// 8192 139, 80, 62, 57; 37 x 4096 x 14336 237, 139, 87, 66; q8_0 131 x 8192 x
+// 2048 37, 28, 30, 31; 131 x 2048 x 8192 124, 77, 62, 44. (16 x 256 and 32 x
+// 256 tiles lost throughout: 213 to 241 VGPRs. A second chunk in flight in
+// registers gained up to 4% at q4_K products of few workgroups and lost 15 to
+// 20% on the other formats, whose scales take more registers.)
 template <int FMT, bool F16S>
 void launch(const MatmulDotArgs& p) {
     const auto waves = [&](uint64_t rt, uint64_t ct) { return ((p.m + 16 * rt - 1) / (16 * rt)) * ((p.n + 16 * ct - 1) / (16 * ct)); };
-    constexpr uint64_t kEnough = 1792;  // 256 CUs x 4 SIMDs x 1.75
-    if (waves(4, 2) >= 4096) {
-        const dim3 grid((p.n + 127) / 128, (p.m + 63) / 64);
-        hipLaunchKernelGGL((k_matmul_dot_staged<FMT, F16S, 4>), grid, dim3(kT), 0, vkml::abi::stream(), p);
-    } else if (waves(2, 2) >= 2048) {
-        const dim3 grid((p.n + 127) / 128, (p.m + 31) / 32);
-        hipLaunchKernelGGL((k_matmul_dot_staged<FMT, F16S, 2>), grid, dim3(kT), 0, vkml::abi::stream(), p);
-    } else if (waves(2, 2) >= 512) {
-        const dim3 grid((p.n + 127) / 128, (p.m + 15) / 16);
-        hipLaunchKernelGGL((k_matmul_dot_staged<FMT, F16S, 1>), grid, dim3(kT), 0, vkml::abi::stream(), p);
-    } else if (waves(2, 2) >= kEnough) launch_tiles<FMT, F16S, 2, 2>(p);
-    else if (waves(2, 1) >= kEnough) launch_tiles<FMT, F16S, 2, 1>(p);
-    else launch_tiles<FMT, F16S, 1, 1>(p);
+    if (waves(4, 2) >= 8192) launch_tile<FMT, F16S, 4, 2>(p);
+    else if (waves(2, 2) >= 1280) launch_tile<FMT, F16S, 2, 2>(p);
+    else if (waves(2, 2) >= 900) launch_tile<FMT, F16S, 1, 2>(p);
+    else launch_tile<FMT, F16S, 1, 1>(p);
 }
 
 int matmul_dot_common(const char* what, const vkml_gemv_dot_params* p, const void* a_values, const void* b_values, float* out,
