@@ -597,6 +597,28 @@ def test_attend_bit_exact(hd, heads, kvh, kv_len, kv_type, extra):
     assert np.array_equal(scs.download(np.float32, ws.shape).view(np.uint32), ws.view(np.uint32))
 
 
+@pytest.mark.parametrize("hd,group,kv_len,kv_type", [
+    (128, 4, 897, H.F16), (128, 4, 1000, H.F32), (64, 4, 1000, H.F16), (64, 8, 900, H.F32),
+    (256, 4, 1000, H.F16), (256, 4, 900, H.F32), (256, 2, 300, H.F16)])
+def test_attend_several_chains_a_thread_bit_exact(hd, group, kv_len, kv_type):
+    # 64 KV heads: enough items for four heads a workgroup at short lengths,
+    # whose V pass gives a thread two or four elements (one from an unstaged
+    # V); whole chunks and a last one of 1, 4, 44 or 104 keys
+    kvh, cap = 64, kv_len + 3
+    heads, chunks = kvh * group, (kv_len + 127) // 128
+    rng = np.random.default_rng(kv_len + hd)
+    q = rng.standard_normal((heads, hd)).astype(np.float32)
+    k = rng.standard_normal((kvh, cap, hd)).astype(np.float32)
+    v = rng.standard_normal((kvh, cap, hd)).astype(np.float32)
+    kc, vc = (k.astype(np.float16).view(np.uint16), v.astype(np.float16).view(np.uint16)) if kv_type == H.F16 else (k, v)
+    prm = H.AttendParams(0, kv_len, cap, heads, kvh, hd, kv_type, chunks, 1.0 / math.sqrt(hd), 0.0)
+    part, stats, out = H.empty(heads * chunks * hd * 4), H.empty(heads * chunks * 8), H.empty(heads * hd * 4)
+    H.call("vkml_attend", prm, p(dev(q)), p(dev(kc)), p(dev(vc)), p(part), p(stats), None)
+    H.call("vkml_attend_merge", prm, p(part), p(stats), p(out), None, None)
+    want = O.attend_decode(q, kc, vc, 0, kv_len)
+    assert np.array_equal(bits(out.download(np.float32, (heads, hd))), bits(want))
+
+
 def test_attend_reads_kv_len_from_the_decode_state():
     hd, heads, kvh, cap = 128, 32, 8, 512
     rng = np.random.default_rng(3)
