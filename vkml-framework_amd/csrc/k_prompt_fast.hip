@@ -10,8 +10,8 @@
 // f32 attention to within f32 rounding.
 //
 // A workgroup takes 16 queries of one KV head's four query heads, a wave a
-// head, and walks the keys its queries see in blocks of 32:
-//   - scores S^T [32 keys x 16 queries] = K . Q^T by
+// head, and walks the keys its queries see in blocks of KB = 32 or 64:
+//   - scores S^T [KB keys x 16 queries] = K . Q^T by
 //     v_mfma_f32_16x16x32_f16, K copied into LDS a block ahead by
 //     global_load_lds (each row's 16-byte pieces swizzled so that the 16
 //     rows of an operand read hit different banks), q (scaled into log2
@@ -19,12 +19,12 @@
 //   - per query (a lane column) the block's max and the running (max, sum),
 //     the accumulated output rescaled by 2^(m_old - m_new);
 //   - O^T [hd x 16 queries] += V^T . P^T, V loaded a block ahead into
-//     registers and written into LDS transposed, [dim][key], so that a
-//     lane's operand is two 8-byte reads; P^T straight from the score
-//     tile's registers (the accumulator layout of S^T is the B operand's
-//     of P^T, keys permuted alike in V^T's A operand). In O^T a query is a
-//     lane column, as in S^T, so its rescale needs no exchange between
-//     lanes.
+//     registers and written into LDS transposed, [dim][key], two keys a
+//     word, so that a lane's operand is two 8-byte reads; P^T straight from
+//     the score tile's registers (the accumulator layout of S^T is the B
+//     operand's of P^T, keys permuted alike in V^T's A operand). In O^T a
+//     query is a lane column, as in S^T, so its rescale needs no exchange
+//     between lanes.
 // The output is written [query, head, hd]: the o projection's input rows.
 #include <algorithm>
 #include <string>
@@ -42,7 +42,6 @@ using vkml::attend_fast::kLog2e;
 namespace {
 
 constexpr uint32_t kQueries = 16;  // queries a workgroup
-constexpr uint32_t kBlock = 32;    // keys a block
 constexpr uint32_t kHeads = 4;     // query heads a workgroup (a wave each)
 
 struct PromptArgs {
@@ -57,59 +56,82 @@ struct PromptArgs {
 // A block's tiles in LDS. K row-major, each row's 16-byte pieces swizzled
 // (piece p of key row r at p ^ (r % pieces)) so that the 16 rows a score
 // operand read takes hit different banks. V transposed, [dim][key] with
-// rows padded to 72 bytes, so that a lane's four keys of one dim are one
+// rows padded to KB + 4 keys, so that a lane's four keys of one dim are one
 // 8-byte read and the 16 dims of a read hit different banks.
-template <int HD>
+template <int HD, int KB>
 struct PromptTiles {
     static constexpr uint32_t kPieces = HD * 2 / 16;  // 16-byte pieces a key row
-    static constexpr uint32_t kVtStride = kBlock + 4;  // f16 a V^T row
-    alignas(16) uint8_t k[kBlock * HD * 2];
+    static constexpr uint32_t kVtStride = KB + 4;      // f16 a V^T row
+    alignas(16) uint8_t k[KB * HD * 2];
     alignas(16) _Float16 vt[HD * kVtStride];
 };
 
-// V of the next block in registers (8 dims of one key a 16-byte piece).
-template <int HD>
+// V of the next block in registers, 8 dims of two consecutive keys an item.
+// An item's wave covers 16 key pairs by 4 pieces of 8 dims: in V^T, whose
+// rows are 18 or 34 words, those 64 lanes' words (a key pair of one dim) lie
+// in 64 different banks. (One key a lane and item, an f16 a store, took
+// twice as many stores and four lanes a bank.)
+template <int HD, int KB>
 struct VRegs {
-    static constexpr uint32_t kLoads = kBlock * HD * 2 / 16 / kThreads;
-    uint4 v[kLoads];
+    static constexpr uint32_t kGroups = (KB / 32) * (HD / 32);  // (16 key pairs, 4 pieces) groups
+    static constexpr uint32_t kWaves = kThreads / kWave;
+    static constexpr uint32_t kItems = (kGroups + kWaves - 1) / kWaves;
+    uint4 v[kItems][2];
+    __device__ static uint32_t group(uint32_t i) { return i * kWaves + thread_index() / kWave; }
+    __device__ static uint32_t pair(uint32_t i) { return group(i) / (HD / 32) * 16 + thread_index() % 16; }
+    __device__ static uint32_t piece(uint32_t i) { return group(i) % (HD / 32) * 4 + thread_index() % kWave / 16; }
 };
 
 // Key block kb's K rows into LDS (global_load_lds, swizzled) and its V rows
 // into registers. Keys past `keys` re-read the last.
-template <int HD>
-__device__ __forceinline__ void load_block(const PromptArgs& a, uint32_t kvh, uint32_t kb, uint32_t keys, PromptTiles<HD>& tl, VRegs<HD>& vr) {
-    using T = PromptTiles<HD>;
+template <int HD, int KB>
+__device__ __forceinline__ void load_block(const PromptArgs& a, uint32_t kvh, uint32_t kb, uint32_t keys, PromptTiles<HD, KB>& tl,
+                                           VRegs<HD, KB>& vr) {
+    using T = PromptTiles<HD, KB>;
+    using V = VRegs<HD, KB>;
     constexpr uint32_t RB = HD * 2;
     const uint32_t t = thread_index(), wave_first = t - t % kWave;
     const uint64_t row0 = static_cast<uint64_t>(kvh) * a.capacity;
     const auto* kc = static_cast<const uint8_t*>(a.k_cache);
     const auto* vc = static_cast<const uint8_t*>(a.v_cache);
+    const auto row_of = [&](uint32_t key) -> uint64_t { return row0 + min(kb * KB + key, keys - 1); };
 #pragma unroll
-    for (uint32_t i = 0; i < VRegs<HD>::kLoads; ++i) {
+    for (uint32_t i = 0; i < KB * RB / 16 / kThreads; ++i) {
         const uint32_t u = i * kThreads + t, rr = u / T::kPieces, piece = u % T::kPieces;
-        const uint64_t row = row0 + min(kb * kBlock + rr, keys - 1);
-        vkml::attend::load_to_lds16(kc + row * RB + 16 * (piece ^ (rr % T::kPieces)), tl.k + 16 * (i * kThreads + wave_first));
-        vr.v[i] = ldg(reinterpret_cast<const uint4*>(vc + row * RB + 16 * piece));
+        vkml::attend::load_to_lds16(kc + row_of(rr) * RB + 16 * (piece ^ (rr % T::kPieces)), tl.k + 16 * (i * kThreads + wave_first));
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < V::kItems; ++i) {
+        if (V::group(i) >= V::kGroups) break;
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e)
+            vr.v[i][e] = ldg(reinterpret_cast<const uint4*>(vc + row_of(2 * V::pair(i) + e) * RB + 16 * V::piece(i)));
     }
 }
 
 // The block's V from registers into its V^T tile.
-template <int HD>
-__device__ __forceinline__ void store_vt(const VRegs<HD>& vr, PromptTiles<HD>& tl) {
-    using T = PromptTiles<HD>;
-    const uint32_t t = thread_index();
+template <int HD, int KB>
+__device__ __forceinline__ void store_vt(const VRegs<HD, KB>& vr, PromptTiles<HD, KB>& tl) {
+    using T = PromptTiles<HD, KB>;
+    using V = VRegs<HD, KB>;
 #pragma unroll
-    for (uint32_t i = 0; i < VRegs<HD>::kLoads; ++i) {
-        const uint32_t u = i * kThreads + t, key = u / T::kPieces, d0 = 8 * (u % T::kPieces);
-        const half8 x = __builtin_bit_cast(half8, vr.v[i]);
+    for (uint32_t i = 0; i < V::kItems; ++i) {
+        if (V::group(i) >= V::kGroups) break;
+        _Float16* to = tl.vt + 8 * V::piece(i) * T::kVtStride + 2 * V::pair(i);
+        const uint4 x = vr.v[i][0], y = vr.v[i][1];
+        const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ys[4] = {y.x, y.y, y.z, y.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) tl.vt[(d0 + e) * T::kVtStride + key] = x[e];
+        for (int e = 0; e < 4; ++e) {
+            *reinterpret_cast<uint32_t*>(to + 2 * e * T::kVtStride) = (xs[e] & 0xFFFFu) | (ys[e] << 16);
+            *reinterpret_cast<uint32_t*>(to + (2 * e + 1) * T::kVtStride) = (xs[e] >> 16) | (ys[e] & 0xFFFF0000u);
+        }
     }
 }
 
-template <int HD>
+template <int HD, int KB>
 __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
-    using T = PromptTiles<HD>;
+    using T = PromptTiles<HD, KB>;
+    constexpr int TT = KB / 16;  // score tiles a block
     __shared__ T s_t[2];
     constexpr int kSteps = HD / 32;
     const uint32_t t = thread_index(), w = t / kWave, l = t % kWave, j = l % 16, g = l / 16;
@@ -126,11 +148,11 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
     const bool qlive = qi < a.t;
     const uint32_t qpos = a.first + min(qi, a.t - 1);                // its position: keys 0 .. qpos
     const uint32_t keys = a.first + min(q0 + kQueries, a.t);         // keys the workgroup's queries see
-    const uint32_t blocks = (keys + kBlock - 1) / kBlock;
+    const uint32_t blocks = (keys + KB - 1) / KB;
     const bool cap = a.softcap > 0.0f;
 
-    VRegs<HD> vr;
-    load_block<HD>(a, kvh, 0, keys, s_t[0], vr);
+    VRegs<HD, KB> vr;
+    load_block<HD, KB>(a, kvh, 0, keys, s_t[0], vr);
     // q of the lane's query, scaled (in log2 units without a soft cap), as hi + lo f16
     half8 qh[kSteps], ql[kSteps];
     {
@@ -167,13 +189,13 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
     // the two tiles (a pair a trip, so each is named statically).
     const auto block = [&](uint32_t kb, T& cur, T& nxt) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's K copies and V loads of block kb have landed
-        store_vt<HD>(vr, cur);
+        store_vt<HD, KB>(vr, cur);
         __syncthreads();  // every wave's; and block kb - 1's tiles are no longer read
-        if (kb + 1 < blocks) load_block<HD>(a, kvh, kb + 1, keys, nxt, vr);
-        // scores: lane (j, g) holds keys 32 kb + 16 tt + 4 g + e of query j
-        f32x4 sacc[2];
+        if (kb + 1 < blocks) load_block<HD, KB>(a, kvh, kb + 1, keys, nxt, vr);
+        // scores: lane (j, g) holds keys KB kb + 16 tt + 4 g + e of query j
+        f32x4 sacc[TT];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+        for (int tt = 0; tt < TT; ++tt) {
             sacc[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             const uint32_t rr = 16 * tt + j;
 #pragma unroll
@@ -184,15 +206,15 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
                 sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[s], sacc[tt], 0, 0, 0);
             }
         }
-        float sc[2][4];
+        float sc[TT][4];
         float bm = -__builtin_inff();
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float x = sacc[tt][e];
                 if (cap) x = a.softcap * tanhf(fminf(fmaxf(x / a.softcap, -10.0f), 10.0f)) * kLog2e;
-                const uint32_t key = kb * kBlock + 16 * tt + 4 * g + e;
+                const uint32_t key = kb * KB + 16 * tt + 4 * g + e;
                 sc[tt][e] = qlive && key <= qpos ? x : -__builtin_inff();
                 bm = fmaxf(bm, sc[tt][e]);
             }
@@ -206,16 +228,16 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
         const bool any = mn != -__builtin_inff();
         const float factor = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
         float bs = 0.0f;
-        half8 ph, pl;
+        half8 ph[TT / 2], pl[TT / 2];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float p = any && sc[tt][e] != -__builtin_inff() ? __builtin_amdgcn_exp2f(sc[tt][e] - mn) : 0.0f;
                 bs += p;
                 const _Float16 hi = static_cast<_Float16>(p);
-                ph[4 * tt + e] = hi;
-                pl[4 * tt + e] = static_cast<_Float16>(p - static_cast<float>(hi));
+                ph[tt / 2][4 * (tt % 2) + e] = hi;
+                pl[tt / 2][4 * (tt % 2) + e] = static_cast<_Float16>(p - static_cast<float>(hi));
             }
         {
             const uint2 a16 = swap_rows<16>(__float_as_uint(bs));
@@ -226,16 +248,19 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
         lsum = lsum * factor + bs;
         m = mn;
         // O^T: lane (j, g) gives V^T at dim 16 dt + j of keys 4 g .. 4 g + 3
-        // and 16 + 4 g .. 16 + 4 g + 3 of the block, the keys its P^T holds
+        // and 16 + 4 g .. 16 + 4 g + 3 of each 32, the keys its P^T holds
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             const _Float16* row = cur.vt + (16 * dt + j) * T::kVtStride + 4 * g;
-            const uint2 lo = *reinterpret_cast<const uint2*>(row), hi = *reinterpret_cast<const uint2*>(row + 16);
-            const half8 va = __builtin_bit_cast(half8, make_uint4(lo.x, lo.y, hi.x, hi.y));
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[dt][e] *= factor;
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph, o[dt], 0, 0, 0);
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl, o[dt], 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < TT / 2; ++u) {
+                const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * u), hi = *reinterpret_cast<const uint2*>(row + 32 * u + 16);
+                const half8 va = __builtin_bit_cast(half8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[u], o[dt], 0, 0, 0);
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[u], o[dt], 0, 0, 0);
+            }
         }
     };
     for (uint32_t kb = 0; kb < blocks; kb += 2) {
@@ -251,6 +276,11 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
             *reinterpret_cast<float4*>(op + 16 * dt) = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
     }
 }
+
+// Past this many keys a block is 64 of them: half the waits, barriers and
+// rescalings of the output a key, more independent matrix instructions
+// between them, against half a block more of masked keys a tile.
+constexpr uint32_t kWideKeys = 128;
 
 const char* check_prompt(const vkml_attend_prompt_params* p) {
     if (!p) return "null params";
@@ -279,10 +309,10 @@ int vkml_attend_prompt_fast(const vkml_attend_prompt_params* p, const float* q, 
                        p->scale, p->softcap};
     const dim3 grid((p->t + kQueries - 1) / kQueries * (p->kv_heads * (a.group / kHeads)));
     vkml::abi::ProfileScope prof("attend_prompt_fast");
-    if (p->head_dim == 128)
-        hipLaunchKernelGGL(k_attend_prompt_fast<128>, grid, dim3(kThreads), 0, vkml::abi::stream(), a);
-    else
-        hipLaunchKernelGGL(k_attend_prompt_fast<64>, grid, dim3(kThreads), 0, vkml::abi::stream(), a);
+    const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, vkml::abi::stream(), a); };
+    const bool wide = p->first + p->t > kWideKeys;
+    if (p->head_dim == 128) wide ? go(k_attend_prompt_fast<128, 64>) : go(k_attend_prompt_fast<128, 32>);
+    else wide ? go(k_attend_prompt_fast<64, 64>) : go(k_attend_prompt_fast<64, 32>);
     return vkml::abi::check_launch("attend_prompt_fast");
 }
 
