@@ -233,6 +233,10 @@ PROMPT_SHAPES = [
     (8, 2, 64, 0, 1000, 1024),
     (16, 2, 128, 5, 130, 200),
     (32, 8, 128, 0, 2048, 2048),
+    # either side of the lines between blocks of 32 and of 64 keys, keys a
+    # whole number of blocks and one more, tiles that start in a later block
+    (8, 2, 64, 0, 64, 64), (8, 2, 64, 1, 64, 70), (32, 8, 128, 0, 192, 192), (8, 2, 128, 3, 190, 200),
+    (4, 1, 128, 240, 17, 257), (8, 1, 128, 63, 193, 256), (32, 8, 128, 0, 1024, 1024), (32, 8, 128, 1, 1025, 1030),
 ]
 
 

@@ -26,6 +26,15 @@
 //     query is a lane column, as in S^T, so its rescale needs no exchange
 //     between lanes.
 // The output is written [query, head, hd]: the o projection's input rows.
+//
+// What bounds it. A tile's blocks follow one another, and few workgroups run
+// beside it: a wave's matrix instructions (64 a 64-key block at head_dim 128,
+// about 0.4 us), its softmax, and the LDS and barrier waits between them take
+// 2.2 us a block. 1000 queries after 37 keys, 32 heads on 8 KV heads of 128:
+// 63.0 us with an f16 a V^T store and 32-key blocks, 43.7 with two keys a
+// store and 64-key blocks, 41.0 with masks only where a tile's queries need
+// them, the output rescaled only when a maximum has moved, and the sums of a
+// query's four lanes added once.
 #include <algorithm>
 #include <string>
 
@@ -181,7 +190,11 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
     f32x4 o[HD / 16];
 #pragma unroll
     for (int dt = 0; dt < HD / 16; ++dt) o[dt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float m = -__builtin_inff(), lsum = 0.0f;  // the lane's query: running max (log2 units) and sum
+    // The lane's query: running max (log2 units) and the sum over the lane's
+    // keys (the query's four lanes' are added at the end). The max starts at
+    // the lowest finite value, so that scores of -inf (masked ones among
+    // them) give 2^(-inf) = 0 whatever came before.
+    float m = -__FLT_MAX__, lsum = 0.0f;
 
     // One block: wait for its loads, put its V into the V^T tile, issue the
     // next block's loads (K into the other tile's LDS, V into registers),
@@ -206,6 +219,9 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
                 sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[s], sacc[tt], 0, 0, 0);
             }
         }
+        // Only the blocks past the tile's first query's position hold keys
+        // that some of its queries don't see.
+        const bool masked = kb * KB + KB > a.first + q0 + 1;
         float sc[TT][4];
         float bm = -__builtin_inff();
 #pragma unroll
@@ -214,10 +230,19 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
             for (int e = 0; e < 4; ++e) {
                 float x = sacc[tt][e];
                 if (cap) x = a.softcap * tanhf(fminf(fmaxf(x / a.softcap, -10.0f), 10.0f)) * kLog2e;
-                const uint32_t key = kb * KB + 16 * tt + 4 * g + e;
-                sc[tt][e] = qlive && key <= qpos ? x : -__builtin_inff();
-                bm = fmaxf(bm, sc[tt][e]);
+                sc[tt][e] = x;
             }
+        if (masked) {
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (kb * KB + 16 * tt + 4 * g + e > qpos) sc[tt][e] = -__builtin_inff();
+        }
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bm = fmaxf(bm, sc[tt][e]);
         {
             const uint2 a16 = swap_rows<16>(__float_as_uint(bm));
             bm = fmaxf(__uint_as_float(a16.x), __uint_as_float(a16.y));
@@ -225,35 +250,33 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
             bm = fmaxf(__uint_as_float(a32.x), __uint_as_float(a32.y));
         }
         const float mn = fmaxf(m, bm);
-        const bool any = mn != -__builtin_inff();
-        const float factor = m == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
+        const float factor = __builtin_amdgcn_exp2f(m - mn);
         float bs = 0.0f;
         half8 ph[TT / 2], pl[TT / 2];
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float p = any && sc[tt][e] != -__builtin_inff() ? __builtin_amdgcn_exp2f(sc[tt][e] - mn) : 0.0f;
+                const float p = __builtin_amdgcn_exp2f(sc[tt][e] - mn);
                 bs += p;
                 const _Float16 hi = static_cast<_Float16>(p);
                 ph[tt / 2][4 * (tt % 2) + e] = hi;
                 pl[tt / 2][4 * (tt % 2) + e] = static_cast<_Float16>(p - static_cast<float>(hi));
             }
-        {
-            const uint2 a16 = swap_rows<16>(__float_as_uint(bs));
-            bs = __uint_as_float(a16.x) + __uint_as_float(a16.y);
-            const uint2 a32 = swap_rows<32>(__float_as_uint(bs));
-            bs = __uint_as_float(a32.x) + __uint_as_float(a32.y);
-        }
         lsum = lsum * factor + bs;
         m = mn;
         // O^T: lane (j, g) gives V^T at dim 16 dt + j of keys 4 g .. 4 g + 3
         // and 16 + 4 g .. 16 + 4 g + 3 of each 32, the keys its P^T holds
+        // (once the maxima have settled, most blocks leave the output's scale)
+        if (__any(factor != 1.0f)) {
+#pragma unroll
+            for (int dt = 0; dt < HD / 16; ++dt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[dt][e] *= factor;
+        }
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt) {
             const _Float16* row = cur.vt + (16 * dt + j) * T::kVtStride + 4 * g;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[dt][e] *= factor;
 #pragma unroll
             for (int u = 0; u < TT / 2; ++u) {
                 const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * u), hi = *reinterpret_cast<const uint2*>(row + 32 * u + 16);
@@ -268,6 +291,10 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
         if (kb + 1 < blocks) block(kb + 1, s_t[1], s_t[0]);
     }
     // lane (j, g) holds dims 16 dt + 4 g .. + 3 of query j
+    const uint2 l16 = swap_rows<16>(__float_as_uint(lsum));
+    lsum = __uint_as_float(l16.x) + __uint_as_float(l16.y);
+    const uint2 l32 = swap_rows<32>(__float_as_uint(lsum));
+    lsum = __uint_as_float(l32.x) + __uint_as_float(l32.y);
     if (qlive) {
         const float inv = 1.0f / lsum;
         float* op = a.out + (static_cast<uint64_t>(qi) * a.heads + h) * HD + 4 * g;
@@ -277,10 +304,19 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
     }
 }
 
-// Past this many keys a block is 64 of them: half the waits, barriers and
-// rescalings of the output a key, more independent matrix instructions
-// between them, against half a block more of masked keys a tile.
-constexpr uint32_t kWideKeys = 128;
+// Whether a block is 64 keys instead of 32: half the waits, barriers and
+// maxima a key and more independent matrix instructions between them, against
+// half a block more of masked keys a tile and twice the LDS, which at head_dim
+// 128 leaves two workgroups a compute unit. Measured (us; 32, 64; 32 heads on
+// 8 KV heads): head_dim 128, 40 queries 5.6, 6.1; 130 8.8, 9.2; 200 11.7,
+// 11.7; 300 16.0, 14.9; 512 23.7, 21.2; 64 after 1000 keys 43.3, 37.9; 1000
+// after 37 44.7, 41.9; 2048 (four workgroups a compute unit) 90.5, 94.3;
+// head_dim 64, 9 queries 3.6, 4.0; 64 after 64 keys 6.2, 5.7; 300 11.2, 9.9;
+// 1000 29.6, 25.7; 2048 after 2048 keys 147, 140.
+bool wide_blocks(const vkml_attend_prompt_params& p, uint32_t workgroups) {
+    const uint32_t keys = p.first + p.t;
+    return p.head_dim == 64 ? keys > 64 : keys > 192 && workgroups <= 2 * vkml::abi::compute_units();
+}
 
 const char* check_prompt(const vkml_attend_prompt_params* p) {
     if (!p) return "null params";
@@ -310,7 +346,7 @@ int vkml_attend_prompt_fast(const vkml_attend_prompt_params* p, const float* q, 
     const dim3 grid((p->t + kQueries - 1) / kQueries * (p->kv_heads * (a.group / kHeads)));
     vkml::abi::ProfileScope prof("attend_prompt_fast");
     const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, vkml::abi::stream(), a); };
-    const bool wide = p->first + p->t > kWideKeys;
+    const bool wide = wide_blocks(*p, grid.x);
     if (p->head_dim == 128) wide ? go(k_attend_prompt_fast<128, 64>) : go(k_attend_prompt_fast<128, 32>);
     else wide ? go(k_attend_prompt_fast<64, 64>) : go(k_attend_prompt_fast<64, 32>);
     return vkml::abi::check_launch("attend_prompt_fast");
