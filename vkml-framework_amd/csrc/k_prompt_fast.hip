@@ -30,11 +30,12 @@
 // What bounds it. A tile's blocks follow one another, and few workgroups run
 // beside it: a wave's matrix instructions (64 a 64-key block at head_dim 128,
 // about 0.4 us), its softmax, and the LDS and barrier waits between them take
-// 2.2 us a block. 1000 queries after 37 keys, 32 heads on 8 KV heads of 128:
+// 2 us a block. 1000 queries after 37 keys, 32 heads on 8 KV heads of 128:
 // 63.0 us with an f16 a V^T store and 32-key blocks, 43.7 with two keys a
 // store and 64-key blocks, 41.0 with masks only where a tile's queries need
 // them, the output rescaled only when a maximum has moved, and the sums of a
-// query's four lanes added once.
+// query's four lanes added once, 37.7 with the matrix instructions of several
+// tiles in turn.
 #include <algorithm>
 #include <string>
 
@@ -208,16 +209,21 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
         // scores: lane (j, g) holds keys KB kb + 16 tt + 4 g + e of query j
         f32x4 sacc[TT];
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-            sacc[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            const uint32_t rr = 16 * tt + j;
+        for (int tt = 0; tt < TT; ++tt) sacc[tt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        // (the block's tiles in turn, so that a matrix instruction does not
+        // wait for the one before it)
 #pragma unroll
-            for (int s = 0; s < kSteps; ++s) {
-                const uint32_t piece = (4 * s + g) ^ (rr % T::kPieces);
-                const half8 kf = *reinterpret_cast<const half8*>(cur.k + rr * (HD * 2) + 16 * piece);
-                sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[s], sacc[tt], 0, 0, 0);
-                sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[s], sacc[tt], 0, 0, 0);
+        for (int s = 0; s < kSteps; ++s) {
+            half8 kf[TT];
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) {
+                const uint32_t rr = 16 * tt + j, piece = (4 * s + g) ^ (rr % T::kPieces);
+                kf[tt] = *reinterpret_cast<const half8*>(cur.k + rr * (HD * 2) + 16 * piece);
             }
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt], qh[s], sacc[tt], 0, 0, 0);
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt) sacc[tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[tt], ql[s], sacc[tt], 0, 0, 0);
         }
         // Only the blocks past the tile's first query's position hold keys
         // that some of its queries don't see.
@@ -274,17 +280,23 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[dt][e] *= factor;
         }
+        constexpr int DT = KB == 64 ? 4 : 2;  // 16-dim tiles in turn, as the scores'
 #pragma unroll
-        for (int dt = 0; dt < HD / 16; ++dt) {
-            const _Float16* row = cur.vt + (16 * dt + j) * T::kVtStride + 4 * g;
+        for (int d0 = 0; d0 < HD / 16; d0 += DT)
 #pragma unroll
             for (int u = 0; u < TT / 2; ++u) {
-                const uint2 lo = *reinterpret_cast<const uint2*>(row + 32 * u), hi = *reinterpret_cast<const uint2*>(row + 32 * u + 16);
-                const half8 va = __builtin_bit_cast(half8, make_uint4(lo.x, lo.y, hi.x, hi.y));
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[u], o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[u], o[dt], 0, 0, 0);
+                half8 va[DT];
+#pragma unroll
+                for (int i = 0; i < DT; ++i) {
+                    const _Float16* row = cur.vt + (16 * (d0 + i) + j) * T::kVtStride + 4 * g + 32 * u;
+                    const uint2 lo = *reinterpret_cast<const uint2*>(row), hi = *reinterpret_cast<const uint2*>(row + 16);
+                    va[i] = __builtin_bit_cast(half8, make_uint4(lo.x, lo.y, hi.x, hi.y));
+                }
+#pragma unroll
+                for (int i = 0; i < DT; ++i) o[d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], ph[u], o[d0 + i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < DT; ++i) o[d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(va[i], pl[u], o[d0 + i], 0, 0, 0);
             }
-        }
     };
     for (uint32_t kb = 0; kb < blocks; kb += 2) {
         block(kb, s_t[0], s_t[1]);
@@ -308,7 +320,7 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
 // maxima a key and more independent matrix instructions between them, against
 // half a block more of masked keys a tile and twice the LDS, which at head_dim
 // 128 leaves two workgroups a compute unit. Measured (us; 32, 64; 32 heads on
-// 8 KV heads): head_dim 128, 40 queries 5.6, 6.1; 130 8.8, 9.2; 200 11.7,
+// 8 KV heads; before the matrix instructions were interleaved): head_dim 128, 40 queries 5.6, 6.1; 130 8.8, 9.2; 200 11.7,
 // 11.7; 300 16.0, 14.9; 512 23.7, 21.2; 64 after 1000 keys 43.3, 37.9; 1000
 // after 37 44.7, 41.9; 2048 (four workgroups a compute unit) 90.5, 94.3;
 // head_dim 64, 9 queries 3.6, 4.0; 64 after 64 keys 6.2, 5.7; 300 11.2, 9.9;
