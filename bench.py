@@ -71,7 +71,7 @@ GATE_UP_TRAFFIC = 67_423_679
 GATE_UP_TRAFFIC_SOURCES = "8ab00a5e354809b3"
 TRAFFIC_FILES = ("vkml-framework_amd/csrc/gemv.hpp", "vkml-framework_amd/csrc/k_gemv.hip", "vkml-framework_amd/csrc/device.hpp")
 ATTEND_TRAFFIC = 28_559_753
-ATTEND_TRAFFIC_SOURCES = "6214fcabee19f834"
+ATTEND_TRAFFIC_SOURCES = "25b8fc154c973f36"
 ATTEND_TRAFFIC_POSITION = 4224  # the launch's shape the figure was taken at (position; 35 chunks, 32 loading early)
 ATTEND_FILES = ("vkml-framework_amd/csrc/k_attend.hip", "vkml-framework_amd/csrc/attend.hpp", "vkml-framework_amd/csrc/gemv.hpp",
                 "vkml-framework_amd/csrc/device.hpp")
