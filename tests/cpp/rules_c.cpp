@@ -1,0 +1,6 @@
+// The dispatch rules of csrc/rules.hpp as C functions, for test_rules.py.
+#include "rules.hpp"
+
+using namespace vkml::rules;
+
+extern "C" int float_loads_c(const vkml_matmul_params* p, uint64_t a, uint64_t b) { return float_loads(*p, a, b); }

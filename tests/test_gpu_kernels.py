@@ -1333,6 +1333,28 @@ def test_matmul_causal_tiles_bit_exact(heads, rows, first):
         assert np.array_equal(bits(o[h]), bits(O.matmul_float(O.T_F32, probs[h], np.ascontiguousarray(kc[0].T), None, hd, keys))), h
 
 
+@pytest.mark.parametrize("transposed", [1, 0])
+def test_matmul_of_a_b_past_2_30_elements(transposed):
+    """The last rows of an f16 b of 2^30 elements and more: its last columns
+    (transposed), or the last of the sums (a's other entries are zeros, which
+    change none), have the bits of a product with those rows alone."""
+    m, cols, rows, tail = 9, 8192, 131072 + 300, 300
+    rng = np.random.default_rng(transposed)
+    last = rng.standard_normal((tail, cols)).astype(np.float16)
+    b = H.empty(rows * cols * 2)
+    H.call("vkml_fill_u32", p(b), 0x3C003C00, rows * cols // 2)
+    H.call("vkml_memcpy_h2d", C.c_void_p(p(b).value + (rows - tail) * cols * 2), last.ctypes.data_as(C.c_void_p), last.nbytes)
+    a = rng.standard_normal((m, cols if transposed else tail)).astype(np.float32)
+    wide = a if transposed else np.concatenate([np.zeros((m, rows - tail), np.float32), a], axis=1)
+    n, k = (rows, cols) if transposed else (cols, rows)
+    out, want = H.empty(m * n * 4), H.empty(m * max(tail, cols) * 4)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, 1, 1, transposed, H.F16, H.F16), p(dev(wide)), p(b), p(out), None)
+    got = out.download(np.float32, (m, n))
+    n, k = (tail, cols) if transposed else (cols, tail)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, 1, 1, transposed, H.F16, H.F16), p(dev(a)), p(dev(last)), p(want), None)
+    assert np.array_equal(bits(got[:, -n:]), bits(want.download(np.float32, (m, n))))
+
+
 @pytest.mark.parametrize("rows,first", [(130, 0), (64, 70), (200, 3)])
 def test_matmul_causal_skip_changes_nothing(rows, first):
     """The causal skip: scores on and below the diagonal (row r sees keys

@@ -1,0 +1,52 @@
+"""The dispatch rules of vkml-framework_amd/csrc/rules.hpp, compiled with the
+host's compiler: which kernel a call takes, without a GPU."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from vkml_amd import hip as H
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+K_SCALAR, K_VEC_B, K_VEC_AB = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rules") / "librules.so")
+    subprocess.run(["g++", "-std=c++20", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I" + os.path.join(ROOT, "vkml-framework_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "cpp", "rules_c.cpp"), "-o", so], check=True)
+    return C.CDLL(so)
+
+
+def _matmul(m, n, k, b_type, transposed, stride=0, batches=1, causal=0, offset=0):
+    return H.MatmulParams(m, n, k, stride, 1, batches, transposed, b_type, H.F16, causal, offset)
+
+
+@pytest.mark.parametrize("b_type", [H.F32, H.F16, H.BF16])
+@pytest.mark.parametrize("m,n,k,transposed", [(16, 151936, 8192, 1), (16, 8192, 151936, 0), (9, 256000, 4096, 1), (9, 300, 1 << 24, 1),
+                                              (2048, 4096, 128, 1), (2048, 128, 4096, 0)])
+def test_aligned_float_products_load_vec4s_at_any_size(rules, b_type, m, n, k, transposed):
+    # b's of 2^30 elements and more and rows past 2^22 among them
+    assert rules.float_loads_c(C.byref(_matmul(m, n, k, b_type, transposed)), C.c_uint64(4096), C.c_uint64(1 << 33)) == K_VEC_AB
+
+
+def test_float_products_off_alignment_load_elements(rules):
+    def loads(p, a=0, b=0):
+        return rules.float_loads_c(C.byref(p), C.c_uint64(a), C.c_uint64(b))
+    for t, n, k in ((1, 7, 8), (0, 8, 7)):
+        assert loads(_matmul(9, n, k, H.F32, t)) == (K_VEC_AB if t else K_VEC_B)
+    assert loads(_matmul(9, 8, 7, H.F16, 1)) == K_SCALAR
+    assert loads(_matmul(9, 7, 8, H.F16, 0)) == K_SCALAR
+    for b_type, unit in ((H.F32, 16), (H.F16, 8), (H.BF16, 8)):
+        for t in (0, 1):
+            p = _matmul(9, 8, 8, b_type, t, stride=64, batches=2)
+            assert loads(p, 32, unit) == K_VEC_AB
+            assert loads(p, 32, unit // 2) == K_SCALAR
+            assert loads(p, 4, unit) == (K_SCALAR if t else K_VEC_B)
+            assert loads(_matmul(9, 8, 8, b_type, t, stride=66, batches=2), 32, unit) == K_SCALAR
+    # a tile's offsets past 32 bits
+    assert loads(_matmul(9, 8, 1 << 25, H.F16, 1)) == K_SCALAR
+    assert loads(_matmul(9, 8, 1 << 25, H.F16, 0)) == K_VEC_B
+    assert loads(_matmul(9, 1 << 25, 8, H.F16, 0)) == K_VEC_B

@@ -35,12 +35,14 @@
 
 #include "device.hpp"
 #include "internal.hpp"
+#include "rules.hpp"
 
 // Products and sums are rounded apart.
 #pragma clang fp contract(off)
 
 using namespace vkml::dev;
 using vkml::abi::ProfileScope;
+using namespace vkml::rules;
 
 namespace {
 
@@ -55,11 +57,6 @@ struct MatmulArgs {
     float* c;
     uint32_t vec_c;  // c's rows are whole, aligned vec4s
 };
-
-// How the operands are loaded: element by element; b four at a time; a and b
-// four at a time (rows of whole, aligned vec4s, and a tile's offsets in 32
-// bits).
-enum Loads { kScalar = 0, kVecB = 1, kVecAB = 2 };
 
 // Four elements of a float b as stored; a quantized b's are widened on load.
 template <uint32_t BTYPE>
@@ -127,8 +124,9 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
     const bool idle = col0 + wave_n >= p.n || row0 + wave_m >= p.m || (BT && p.causal && col0 + wave_n > last_key);
     // The operands: a's rows from row0, b's batch.
     const float* a0 = g.a + (static_cast<uint64_t>(z) * p.m + row0) * p.k;
-    const uint64_t b0 = static_cast<uint64_t>(z / p.b_group) * p.b_stride;
+    const uint64_t b0 = static_cast<uint64_t>(z / p.b_group) * p.b_stride + (BT ? static_cast<uint64_t>(col0) * p.k : 0);
     using Off = std::conditional_t<LOADS == kVecAB, uint32_t, uint64_t>;
+    constexpr bool kChunkBase = !BT && LOADS == kVecAB;  // offsets of a b [k, n] from the chunk's first row
 
     // Every load of a chunk is issued without a branch (indices past the
     // operands re-read their last elements: rows and columns past the end
@@ -153,17 +151,19 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
 #pragma unroll
         for (uint32_t u = 0; u < NB; ++u) {
             const uint32_t e = t + kT * u;
-            // four elements along the rows of b: `from` of a row of `len`
-            const uint32_t line = BT ? min(col0 + e / (kKB / 4), p.n - 1) : min(k0 + e / (TN / 4), p.k - 1);
+            // four elements along the rows of b: `from` of a row of `len`, the
+            // tile's row `line` (of a b [k, n] the chunk's, or b's)
+            const uint32_t line0 = BT || kChunkBase ? 0 : k0;
+            const uint32_t line = BT ? min(e / (kKB / 4), p.n - 1 - col0) : min(line0 + e / (TN / 4), p.k - 1 - (k0 - line0));
             const uint32_t from = BT ? k0 + 4 * (e % (kKB / 4)) : col0 + 4 * (e % (TN / 4)), len = BT ? p.k : p.n;
             if constexpr (BTYPE >= VKML_Q8_0) {
                 float v[4];
 #pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) v[i] = weight_value(BTYPE, p.scale_type, g.b, g.bs, p.k, line, min(from + i, p.k - 1));
+                for (uint32_t i = 0; i < 4; ++i) v[i] = weight_value(BTYPE, p.scale_type, g.b, g.bs, p.k, col0 + line, min(from + i, p.k - 1));
                 rb[u] = make_float4(v[0], v[1], v[2], v[3]);
             } else {
                 using E = std::conditional_t<BTYPE == VKML_F32, float, uint16_t>;
-                const E* base = static_cast<const E*>(g.b) + b0;
+                const E* base = static_cast<const E*>(g.b) + b0 + (kChunkBase ? static_cast<uint64_t>(k0) * p.n : 0);
                 const Off at = static_cast<Off>(line) * len;
                 if constexpr (LOADS != kScalar) {
                     rb[u] = *reinterpret_cast<const BRaw<BTYPE>*>(base + (at + min(from, len - 4)));
@@ -334,16 +334,10 @@ void launch(const MatmulArgs& g) {
 
 template <uint32_t BTYPE>
 void launch_float(const MatmulArgs& g) {
-    const vkml_matmul_params& p = g.p;
-    const bool t = p.b_transposed != 0;
-    // Whole, aligned vec4s along k in a's rows; along k in a transposed b's
-    // rows, along n in b's otherwise. (And a tile's offsets fit 32 bits.)
-    const uint32_t len = t ? p.k : p.n;
-    const bool vec_a = p.k % 4 == 0 && reinterpret_cast<uintptr_t>(g.a) % 16 == 0 && p.k < (1u << 22) && static_cast<uint64_t>(p.k) * p.n < (1ull << 30);
-    const bool vec_b = len % 4 == 0 && p.b_stride % 4 == 0 && reinterpret_cast<uintptr_t>(g.b) % (BTYPE == VKML_F32 ? 16 : 8) == 0;
-    if (t) vec_a && vec_b ? launch<true, BTYPE, kVecAB>(g) : launch<true, BTYPE, kScalar>(g);
-    else if (vec_b) vec_a ? launch<false, BTYPE, kVecAB>(g) : launch<false, BTYPE, kVecB>(g);
-    else launch<false, BTYPE, kScalar>(g);
+    const Loads loads = vkml::rules::float_loads(g.p, reinterpret_cast<uintptr_t>(g.a), reinterpret_cast<uintptr_t>(g.b));
+    if (g.p.b_transposed) loads == kVecAB ? launch<true, BTYPE, kVecAB>(g) : launch<true, BTYPE, kScalar>(g);
+    else if (loads == kVecAB) launch<false, BTYPE, kVecAB>(g);
+    else loads == kVecB ? launch<false, BTYPE, kVecB>(g) : launch<false, BTYPE, kScalar>(g);
 }
 
 }  // namespace
