@@ -1355,6 +1355,27 @@ def test_matmul_of_a_b_past_2_30_elements(transposed):
     assert np.array_equal(bits(got[:, -n:]), bits(want.download(np.float32, (m, n))))
 
 
+@pytest.mark.parametrize("transposed", [1, 0])
+@pytest.mark.parametrize("batches,m,n", [(32, 530, 2052), (16, 530, 1028), (8, 401, 1004), (2, 17, 68)])
+@pytest.mark.parametrize("k", [4, 8, 9, 16, 24, 31, 40, 48, 57, 64, 80, 88, 95])
+def test_matmul_last_chunk_lengths_bit_exact(transposed, batches, m, n, k):
+    """Every wave tile's last chunk of k's, cut after each number of steps:
+    the same bits with infinities and NaN in a and in b past the k's that are
+    summed (rows of the next matrix), which no product may reach."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((batches * m + 64, k)).astype(np.float32)
+    a[batches * m:] = np.inf
+    b = rng.standard_normal((n if transposed else k, k if transposed else n)).astype(np.float32)
+    past = np.full((64,) + b.shape[1:], np.nan, np.float32)
+    out = H.empty(batches * m * n * 4)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, batches, batches, transposed, H.F32, H.F16), p(dev(a)), p(dev(np.concatenate([b, past]))), p(out), None)
+    got = out.download(np.float32, (batches, m, n))
+    z = batches - 1
+    rows = np.unique(np.concatenate([np.arange(min(m, 8)), np.arange(max(m - 8, 0), m), np.arange(0, m, 37)]))
+    want = O.matmul_float(O.T_F32, a[z * m + rows], b if transposed else np.ascontiguousarray(b.T), None, n, k)
+    assert np.array_equal(bits(got[z][rows]), bits(want))
+
+
 @pytest.mark.parametrize("rows,first", [(130, 0), (64, 70), (200, 3)])
 def test_matmul_causal_skip_changes_nothing(rows, first):
     """The causal skip: scores on and below the diagonal (row r sees keys
