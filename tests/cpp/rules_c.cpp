@@ -4,3 +4,6 @@
 using namespace vkml::rules;
 
 extern "C" int float_loads_c(const vkml_matmul_params* p, uint64_t a, uint64_t b) { return float_loads(*p, a, b); }
+
+// 10 r + nc
+extern "C" int wave_tile_c(const vkml_matmul_params* p) { return 10 * wave_tile(*p).r + wave_tile(*p).nc; }

@@ -1376,6 +1376,30 @@ def test_matmul_last_chunk_lengths_bit_exact(transposed, batches, m, n, k):
     assert np.array_equal(bits(got[z][rows]), bits(want))
 
 
+@pytest.mark.parametrize("fmt,f16", [(H.Q8_0, True), (H.Q8_0, False), (H.Q4_0, True), (H.Q4_0, False), (H.Q4_1, True), (H.Q4_1, False), (H.Q4_K, True)])
+@pytest.mark.parametrize("m,n,k", [(9, 70, 256), (17, 33, 512), (1030, 2050, 256), (1050, 8200, 96), (1050, 31800, 32)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_matmul_quantized_tiles_bit_exact(fmt, f16, m, n, k, shift):
+    """The four wave tiles of a quantized b (three of q4_K) with ragged rows
+    and columns, f16 and f32 scales, an a that starts off alignment, and q8_0
+    and q4_K codes that start at an odd byte."""
+    if fmt == H.Q4_K:
+        k = 256 * (-(-k // 256))
+    v, s, quant, words, scales = weights(fmt, n, k, m + n, f16_scales=f16)
+    if shift and fmt in (H.Q8_0, H.Q4_K):
+        raw = v.download(np.uint8, (v.nbytes,))
+        v = dev(np.concatenate([np.zeros(3, np.uint8), raw]))
+    at = C.c_void_p(p(v).value + (3 if shift and fmt in (H.Q8_0, H.Q4_K) else 0))
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    da = dev(np.concatenate([np.zeros(shift, np.float32), a.ravel()]))
+    out = H.empty(m * n * 4)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, 1, 1, 1, fmt, H.F16 if f16 else H.F32), C.c_void_p(p(da).value + 4 * shift), at, p(out), p(s))
+    got = out.download(np.float32, (m, n))
+    rows = np.unique(np.concatenate([np.arange(min(m, 8)), np.arange(max(m - 8, 0), m), np.arange(0, m, 131)]))
+    want = O.matmul_float({O.Q8_0: O.T_Q8, O.Q4_0: O.T_Q4, O.Q4_1: O.T_Q4_1}[quant], a[rows], words, scales, n, k)
+    assert np.array_equal(bits(got[rows]), bits(want))
+
+
 @pytest.mark.parametrize("rows,first", [(130, 0), (64, 70), (200, 3)])
 def test_matmul_causal_skip_changes_nothing(rows, first):
     """The causal skip: scores on and below the diagonal (row r sees keys

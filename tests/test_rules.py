@@ -50,3 +50,24 @@ def test_float_products_off_alignment_load_elements(rules):
     assert loads(_matmul(9, 8, 1 << 25, H.F16, 1)) == K_SCALAR
     assert loads(_matmul(9, 8, 1 << 25, H.F16, 0)) == K_VEC_B
     assert loads(_matmul(9, 1 << 25, 8, H.F16, 0)) == K_VEC_B
+
+
+# us of vkml_matmul with each wave tile (32 x 64, 32 x 32, 16 x 32, 16 x 16)
+QUANT_TILES = [
+    (H.Q4_K, 9, 4096, 4096, (585, 283, 189, 113)), (H.Q4_K, 64, 8192, 2048, (292, 144, 97.5, 70.8)),
+    (H.Q4_K, 131, 8192, 2048, (297, 190, 158, 146)), (H.Q4_K, 200, 4096, 4096, (599, 289, 232, 227)),
+    (H.Q4_K, 300, 4096, 4096, (603, 382, 316, 292)), (H.Q4_K, 300, 8192, 2048, (383, 270, 234, 259)),
+    (H.Q4_K, 512, 2048, 2048, (304, 148, 121, 118)), (H.Q4_K, 512, 4096, 4096, (611, 383, 387, 418)),
+    (H.Q4_K, 512, 8192, 2048, (387, 335, 350, 401)), (H.Q4_K, 1000, 2048, 2048, (309, 193, 195, 211)),
+    (H.Q4_K, 2048, 14336, 4096, (4244, 4109, None, None)), (H.Q4_K, 4096, 14336, 1024, (2085, 2048, None, None)),
+    (H.Q4_1, 512, 4096, 4096, (512, 365, 375, 382)), (H.Q4_1, 512, 8192, 2048, (331, 321, 346, 361)),
+    (H.Q4_1, 200, 8192, 2048, (259, 183, 187, 171)), (H.Q4_1, 4096, 14336, 1024, (1946, 2000, None, None)),
+    (H.Q8_0, 512, 8192, 2048, (337, 324, 321, 349)), (H.Q8_0, 300, 8192, 2048, (337, 263, 219, 229)),
+    (H.Q8_0, 2048, 14336, 4096, (3879, 3984, None, None)), (H.Q4_0, 300, 8192, 2048, (321, 259, 231, 222)),
+]
+
+
+@pytest.mark.parametrize("b_type,m,n,k,us", QUANT_TILES)
+def test_quantized_products_take_a_tile_within_5_percent_of_the_fastest(rules, b_type, m, n, k, us):
+    picked = (42, 22, 21, 11).index(rules.wave_tile_c(C.byref(_matmul(m, n, k, b_type, 1))))
+    assert us[picked] <= 1.05 * min(u for u in us if u)

@@ -354,6 +354,18 @@ __device__ __forceinline__ void q4k_scales(uint4 hdr, uint32_t c, float& s0, flo
     o1 = round_to_f16(-(dmin * static_cast<float>(mn >> 8)));
 }
 
+// The same of sub-block j alone.
+__device__ __forceinline__ void q4k_block_scale(const uint4& h, uint32_t j, float& s, float& o) {
+    const uint32_t b = 8 * (j % 4);
+    const uint32_t b1 = (h.y >> b) & 0xFFu, b2 = (h.z >> b) & 0xFFu, b3 = (h.w >> b) & 0xFFu;
+    const uint32_t sc = j < 4 ? b1 & 63u : (b3 & 15u) | ((b1 >> 6) << 4);
+    const uint32_t mn = j < 4 ? b2 & 63u : (b3 >> 4) | ((b2 >> 6) << 4);
+    const _Float16 d = __builtin_bit_cast(_Float16, static_cast<uint16_t>(h.x & 0xFFFFu));
+    const _Float16 nd = -__builtin_bit_cast(_Float16, static_cast<uint16_t>(h.x >> 16));
+    s = static_cast<float>(d * static_cast<_Float16>(static_cast<uint16_t>(sc)));
+    o = static_cast<float>(nd * static_cast<_Float16>(static_cast<uint16_t>(mn)));
+}
+
 // Bit offset of value i % 8 within a QuantizedMatrix q4 word
 // (shaders/include/halves.glsl:27).
 __device__ __forceinline__ uint32_t q4_shift(uint32_t i) { return 8u * (i & 3u) + 4u * ((i >> 2) & 1u); }

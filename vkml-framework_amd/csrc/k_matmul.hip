@@ -95,19 +95,6 @@ __device__ __forceinline__ void b_block_scale(const MatmulDotArgs& p, uint32_t n
     }
 }
 
-// q4_K: sub-block j's scale f16(d sc_j) and offset f16(-dmin m_j) from the
-// super-block's 16-byte header (gguf.cpp:603-617).
-__device__ __forceinline__ void q4k_block_scale(const uint4& h, uint32_t j, float& s, float& o) {
-    const uint32_t b = 8 * (j % 4);
-    const uint32_t b1 = (h.y >> b) & 0xFFu, b2 = (h.z >> b) & 0xFFu, b3 = (h.w >> b) & 0xFFu;
-    const uint32_t sc = j < 4 ? b1 & 63u : (b3 & 15u) | ((b1 >> 6) << 4);
-    const uint32_t mn = j < 4 ? b2 & 63u : (b3 >> 4) | ((b2 >> 6) << 4);
-    const _Float16 d = __builtin_bit_cast(_Float16, static_cast<uint16_t>(h.x & 0xFFFFu));
-    const _Float16 nd = -__builtin_bit_cast(_Float16, static_cast<uint16_t>(h.x >> 16));
-    s = static_cast<float>(d * static_cast<_Float16>(static_cast<uint16_t>(sc)));
-    o = static_cast<float>(nd * static_cast<_Float16>(static_cast<uint16_t>(mn)));
-}
-
 constexpr uint32_t kChunk = 8;  // blocks of K a chunk (a q4_K super-block)
 
 // The offset formats with f16 scales (q4_K, q4_1 with f16 scales) take the

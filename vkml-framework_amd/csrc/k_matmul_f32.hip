@@ -58,16 +58,88 @@ struct MatmulArgs {
     uint32_t vec_c;  // c's rows are whole, aligned vec4s
 };
 
-// Four elements of a float b as stored; a quantized b's are widened on load.
+// Four elements of b as stored, along its rows (so of one block of a
+// quantized b): floats; or the codes' word and their scale and offset, f16 or
+// f32 bits, or q4_K header. They are widened when they are staged, so that a
+// chunk's loads wait for nothing.
 template <uint32_t BTYPE>
-using BRaw = std::conditional_t<BTYPE == VKML_F16 || BTYPE == VKML_BF16, uint2, float4>;
+struct BRaw {
+    uint32_t codes, scale, offset;
+};
+template <>
+struct BRaw<VKML_Q4_K> {
+    uint32_t codes;
+    uint4 header;
+};
+template <>
+struct BRaw<VKML_F32> {
+    float4 v;
+};
+template <>
+struct BRaw<VKML_F16> {
+    uint2 v;
+};
+template <>
+struct BRaw<VKML_BF16> {
+    uint2 v;
+};
 
+// Elements col .. col + 3 (col a multiple of 4) of row `row` of a quantized b
+// [rows, cols].
 template <uint32_t BTYPE>
-__device__ __forceinline__ float4 widen(BRaw<BTYPE> w) {
-    if constexpr (BTYPE == VKML_F16 || BTYPE == VKML_BF16)
-        return make_float4(half_to_float(w.x & 0xFFFFu, BTYPE), half_to_float(w.x >> 16, BTYPE), half_to_float(w.y & 0xFFFFu, BTYPE),
-                           half_to_float(w.y >> 16, BTYPE));
-    else return w;
+__device__ __forceinline__ BRaw<BTYPE> load_codes(const MatmulArgs& g, uint64_t row, uint32_t col) {
+    const uint64_t cols = g.p.k, e = row * cols + col;
+    BRaw<BTYPE> r{};
+    if constexpr (BTYPE == VKML_Q4_K) {
+        // sub-block j of the super-block: the low or the high nibbles of bytes 32 (j / 2) ..
+        const uint32_t j = col % 256 / 32;
+        __builtin_memcpy(&r.codes, static_cast<const uint8_t*>(g.b) + row * (cols / 2) + col / 256 * 128 + 32 * (j / 2) + col % 32, 4);
+        r.header = static_cast<const uint4*>(g.bs)[row * (cols / 256) + col / 256];
+    } else {
+        if constexpr (BTYPE == VKML_Q8_0) __builtin_memcpy(&r.codes, static_cast<const uint8_t*>(g.b) + e, 4);
+        else r.codes = static_cast<const uint32_t*>(g.b)[e / 8];
+        constexpr uint32_t per = BTYPE == VKML_Q4_1 ? 2 : 1;
+        const uint64_t at = e / 32 * per;
+        if (g.p.scale_type == VKML_F16) {
+            r.scale = static_cast<const uint16_t*>(g.bs)[at];
+            if constexpr (per == 2) r.offset = static_cast<const uint16_t*>(g.bs)[at + 1];
+        } else {
+            r.scale = static_cast<const uint32_t*>(g.bs)[at];
+            if constexpr (per == 2) r.offset = static_cast<const uint32_t*>(g.bs)[at + 1];
+        }
+    }
+    return r;
+}
+
+// The four elements' values (weight_value's), col their place in the row.
+template <uint32_t BTYPE>
+__device__ __forceinline__ float4 widen(const BRaw<BTYPE>& w, uint32_t col, uint32_t scale_type) {
+    if constexpr (BTYPE == VKML_F32) {
+        return w.v;
+    } else if constexpr (BTYPE == VKML_F16 || BTYPE == VKML_BF16) {
+        return make_float4(half_to_float(w.v.x & 0xFFFFu, BTYPE), half_to_float(w.v.x >> 16, BTYPE), half_to_float(w.v.y & 0xFFFFu, BTYPE),
+                           half_to_float(w.v.y >> 16, BTYPE));
+    } else {
+        float s, o = 0.0f, v[4];
+        if constexpr (BTYPE == VKML_Q4_K) {
+            q4k_block_scale(w.header, col % 256 / 32, s, o);
+        } else {
+            s = scale_type == VKML_F16 ? f16_bits_to_float(static_cast<uint16_t>(w.scale)) : __uint_as_float(w.scale);
+            if constexpr (BTYPE == VKML_Q4_1) o = scale_type == VKML_F16 ? f16_bits_to_float(static_cast<uint16_t>(w.offset)) : __uint_as_float(w.offset);
+        }
+        const uint32_t half = BTYPE == VKML_Q4_K ? col % 64 / 32 : col % 8 / 4;  // low or high nibbles
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            if constexpr (BTYPE == VKML_Q8_0) {
+                v[i] = static_cast<float>(static_cast<int8_t>(w.codes >> (8 * i))) * s;
+            } else {
+                const uint32_t q = (w.codes >> (8 * i + 4 * half)) & 15u;
+                if constexpr (BTYPE == VKML_Q4_0) v[i] = static_cast<float>(static_cast<int>(q) - 8) * s;
+                else v[i] = static_cast<float>(q) * s + o;
+            }
+        }
+        return make_float4(v[0], v[1], v[2], v[3]);
+    }
 }
 
 // v with the elements from i on that are not below end set to zero.
@@ -157,21 +229,18 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
             const uint32_t line = BT ? min(e / (kKB / 4), p.n - 1 - col0) : min(line0 + e / (TN / 4), p.k - 1 - (k0 - line0));
             const uint32_t from = BT ? k0 + 4 * (e % (kKB / 4)) : col0 + 4 * (e % (TN / 4)), len = BT ? p.k : p.n;
             if constexpr (BTYPE >= VKML_Q8_0) {
-                float v[4];
-#pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) v[i] = weight_value(BTYPE, p.scale_type, g.b, g.bs, p.k, col0 + line, min(from + i, p.k - 1));
-                rb[u] = make_float4(v[0], v[1], v[2], v[3]);
+                rb[u] = load_codes<BTYPE>(g, col0 + line, min(from, p.k - 4));
             } else {
                 using E = std::conditional_t<BTYPE == VKML_F32, float, uint16_t>;
                 const E* base = static_cast<const E*>(g.b) + b0 + (kChunkBase ? static_cast<uint64_t>(k0) * p.n : 0);
                 const Off at = static_cast<Off>(line) * len;
                 if constexpr (LOADS != kScalar) {
-                    rb[u] = *reinterpret_cast<const BRaw<BTYPE>*>(base + (at + min(from, len - 4)));
+                    rb[u].v = *reinterpret_cast<const decltype(rb[u].v)*>(base + (at + min(from, len - 4)));
                 } else {
                     const E* src = base + at;
                     const E e0 = src[min(from, len - 1)], e1 = src[min(from + 1, len - 1)], e2 = src[min(from + 2, len - 1)], e3 = src[min(from + 3, len - 1)];
-                    if constexpr (BTYPE == VKML_F32) rb[u] = make_float4(e0, e1, e2, e3);
-                    else rb[u] = make_uint2(e0 | (static_cast<uint32_t>(e1) << 16), e2 | (static_cast<uint32_t>(e3) << 16));
+                    if constexpr (BTYPE == VKML_F32) rb[u].v = make_float4(e0, e1, e2, e3);
+                    else rb[u].v = make_uint2(e0 | (static_cast<uint32_t>(e1) << 16), e2 | (static_cast<uint32_t>(e3) << 16));
                 }
             }
         }
@@ -202,7 +271,7 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
 #pragma unroll
         for (uint32_t u = 0; u < NB; ++u) {
             const uint32_t e = t + kT * u;
-            const float4 v = widen<BTYPE>(rb[u]);
+            const float4 v = widen<BTYPE>(rb[u], BT ? k0 + 4 * (e % (kKB / 4)) : 0, p.scale_type);
             if constexpr (BT) {
                 const uint32_t kq = e % (kKB / 4);
                 put(tb + (e / (kKB / 4)) * kStr, kq, tail ? keep_below(v, k0 + 4 * kq, k_end) : v);
@@ -315,24 +384,11 @@ void launch_tile(const MatmulArgs& g) {
 
 template <bool BT, uint32_t BTYPE, int LOADS>
 void launch(const MatmulArgs& g) {
-    // Waves with work at a wave tile of 16 nc rows by 16 r columns: under a
-    // causal mask the part of the keys that the average query sees.
-    const vkml_matmul_params& p = g.p;
-    const double seen = p.causal ? (p.causal_offset + 0.5 * p.m) / (p.causal_offset + 1.0 * p.m) : 1.0;
-    const auto waves = [&](uint64_t r, uint64_t nc) {
-        return seen * static_cast<double>((p.m + 16 * nc - 1) / (16 * nc) * ((p.n + 16 * r - 1) / (16 * r)) * p.batches);
-    };
-    // The larger a tile, the fewer operands it stages; the smaller, the more
-    // waves and the less padding. Measured (us; wave tiles of 32 x 64, 32 x
-    // 32, 16 x 32 and 16 x 16): scores of 2048 queries by 4096 keys, 32 heads
-    // of 128, 996, 1015, 1107, 1249; 8192 x 8192 x 128 295, 298, 329, 376;
-    // 2048 x 8192 x 2048 1111, 1095, 1155, 1275; probs v at those 2048
-    // queries 952, 909, 942, 1014; 900 x 8192 x 2048 603, 576, 556, 588;
-    // 200 x 14336 x 4096 626, 587, 533, 499; 131 x 2048 x 8192 886, 471, 283,
-    // 218.
-    if (waves(4, 2) >= 16384) launch_tile<BT, BTYPE, LOADS, 4, 2>(g);
-    else if (waves(2, 2) >= 8192) launch_tile<BT, BTYPE, LOADS, 2, 2>(g);
-    else if (waves(2, 1) >= 6144) launch_tile<BT, BTYPE, LOADS, 2, 1>(g);
+    const WaveTile tile = wave_tile(g.p);
+    if constexpr (BTYPE != VKML_Q4_K) {
+        if (tile.r == 4) return launch_tile<BT, BTYPE, LOADS, 4, 2>(g);
+    }
+    if (tile.r == 2) tile.nc == 2 ? launch_tile<BT, BTYPE, LOADS, 2, 2>(g) : launch_tile<BT, BTYPE, LOADS, 2, 1>(g);
     else launch_tile<BT, BTYPE, LOADS, 1, 1>(g);
 }
 
@@ -342,6 +398,11 @@ void launch_float(const MatmulArgs& g) {
     if (g.p.b_transposed) loads == kVecAB ? launch<true, BTYPE, kVecAB>(g) : launch<true, BTYPE, kScalar>(g);
     else if (loads == kVecAB) launch<false, BTYPE, kVecAB>(g);
     else loads == kVecB ? launch<false, BTYPE, kVecB>(g) : launch<false, BTYPE, kScalar>(g);
+}
+
+template <uint32_t BTYPE>
+void launch_quant(const MatmulArgs& g) {
+    quant_loads(g.p, reinterpret_cast<uintptr_t>(g.a)) == kVecAB ? launch<true, BTYPE, kVecAB>(g) : launch<true, BTYPE, kScalar>(g);
 }
 
 }  // namespace
@@ -374,10 +435,10 @@ extern "C" int vkml_matmul(const vkml_matmul_params* p, const float* a, const vo
         case VKML_F32: launch_float<VKML_F32>(g); break;
         case VKML_F16: launch_float<VKML_F16>(g); break;
         case VKML_BF16: launch_float<VKML_BF16>(g); break;
-        case VKML_Q8_0: launch<true, VKML_Q8_0, kScalar>(g); break;
-        case VKML_Q4_0: launch<true, VKML_Q4_0, kScalar>(g); break;
-        case VKML_Q4_1: launch<true, VKML_Q4_1, kScalar>(g); break;
-        default: launch<true, VKML_Q4_K, kScalar>(g); break;
+        case VKML_Q8_0: launch_quant<VKML_Q8_0>(g); break;
+        case VKML_Q4_0: launch_quant<VKML_Q4_0>(g); break;
+        case VKML_Q4_1: launch_quant<VKML_Q4_1>(g); break;
+        default: launch_quant<VKML_Q4_K>(g); break;
     }
     return vkml::abi::check_launch("matmul");
 }

@@ -27,4 +27,40 @@ inline Loads float_loads(const vkml_matmul_params& p, uintptr_t a, uintptr_t b) 
     return vec_b && !p.b_transposed ? kVecB : kScalar;
 }
 
+// A quantized b's codes come four at a time whatever their address; a's
+// loads follow a's alignment (k is whole blocks).
+inline Loads quant_loads(const vkml_matmul_params& p, uintptr_t a) { return a % 16 == 0 && p.k < (1u << 25) ? kVecAB : kScalar; }
+
+// A wave's tile of the product: 16 nc rows by 16 r columns.
+struct WaveTile {
+    int r, nc;
+};
+
+// The larger a tile, the fewer operands it stages; the smaller, the more
+// waves and the less padding. The lines are at the waves with work that a
+// tile gives; under a causal mask the part of the keys that the average query
+// sees. Measured (us; wave tiles of 32 x 64, 32 x 32, 16 x 32 and 16 x 16):
+// scores of 2048 queries by 4096 keys, 32 heads of 128, 996, 1015, 1107, 1249;
+// 8192 x 8192 x 128 295, 298, 329, 376; 2048 x 8192 x 2048 1111, 1095, 1155,
+// 1275; probs v at those 2048 queries 952, 909, 942, 1014; 900 x 8192 x 2048
+// 603, 576, 556, 588; 200 x 14336 x 4096 626, 587, 533, 499; 131 x 2048 x
+// 8192 886, 471, 283, 218. Every tile of columns widens a quantized b again,
+// so the taller tiles win from fewer waves on: q4_K 512 x 8192 x 2048 387,
+// 335, 350, 401; 512 x 4096 x 4096 611, 383, 387, 418; 1000 x 2048 x 2048 309,
+// 193, 195, 211; 300 x 8192 x 2048 383, 270, 234, 259; 131 x 8192 x 2048 297,
+// 190, 158, 146; q4_0 2048 x 14336 x 4096 3846, 3924, -, -. The q4_K 32 x 64
+// tile, whose headers take the registers that its loads would be in flight in,
+// loses everywhere (2048 x 14336 x 4096 4244 against 4109).
+inline WaveTile wave_tile(const vkml_matmul_params& p) {
+    const double seen = p.causal ? (p.causal_offset + 0.5 * p.m) / (p.causal_offset + 1.0 * p.m) : 1.0;
+    const auto waves = [&](uint64_t r, uint64_t nc) {
+        return seen * static_cast<double>((p.m + 16 * nc - 1) / (16 * nc) * ((p.n + 16 * r - 1) / (16 * r)) * p.batches);
+    };
+    const bool quant = p.b_type >= VKML_Q8_0;
+    if (p.b_type != VKML_Q4_K && waves(4, 2) >= 16384) return {4, 2};
+    if (waves(2, 2) >= (quant ? 3072 : 8192)) return {2, 2};
+    if (waves(2, 1) >= (quant ? 3584 : 6144)) return {2, 1};
+    return {1, 1};
+}
+
 }  // namespace vkml::rules
