@@ -7,3 +7,5 @@ extern "C" int float_loads_c(const vkml_matmul_params* p, uint64_t a, uint64_t b
 
 // 10 r + nc
 extern "C" int wave_tile_c(const vkml_matmul_params* p) { return 10 * wave_tile(*p).r + wave_tile(*p).nc; }
+
+extern "C" int cut_last_chunk_c(const vkml_matmul_params* p) { return cut_last_chunk(*p); }

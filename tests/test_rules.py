@@ -71,3 +71,11 @@ QUANT_TILES = [
 def test_quantized_products_take_a_tile_within_5_percent_of_the_fastest(rules, b_type, m, n, k, us):
     picked = (42, 22, 21, 11).index(rules.wave_tile_c(C.byref(_matmul(m, n, k, b_type, 1))))
     assert us[picked] <= 1.05 * min(u for u in us if u)
+
+
+def test_short_sums_that_end_in_a_chunks_first_half_are_cut(rules):
+    def cut(k, b_type=H.F16, t=1):
+        return bool(rules.cut_last_chunk_c(C.byref(_matmul(512, 512, k, b_type, t))))
+    assert all(cut(k, b) for k in (1, 16, 72, 80, 144, 240) for b in (H.F32, H.F16, H.BF16))
+    assert not any(cut(k) for k in (17, 32, 64, 96, 120, 128, 256, 272, 2064))  # (whole chunks and long sums lose by it)
+    assert not cut(80, t=0)

@@ -153,7 +153,7 @@ __host__ __device__ __forceinline__ uint32_t visible_tiles(const vkml_matmul_par
     return static_cast<uint32_t>(last_key < p.n - 1 ? last_key : p.n - 1) / tn + 1;
 }
 
-template <bool BT, uint32_t BTYPE, int R, int NC, int LOADS>
+template <bool BT, uint32_t BTYPE, int R, int NC, int LOADS, bool CUT>
 __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
     constexpr uint32_t KK = 4 / R;                 // k's an instruction
     constexpr uint32_t WR = R == 1 ? 1 : 2;        // waves along the rows
@@ -311,10 +311,9 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
         __syncthreads();
         if (k0 + kKB < k_end) load(k0 + kKB);
         if (idle) continue;
-        // The last chunk's k's past the sums are left out, two steps at a time
-        // (not in the smallest tile, whose chain of chunks a loop of other
-        // than constant length makes 4 to 10% longer).
-        const uint32_t end = R == 1 ? PK / 4 : min(PK / 4, 2 * ((k_end - k0 + 8 * KK - 1) / (8 * KK)));
+        // CUT: the last chunk's k's past the sums are left out, two steps at a
+        // time.
+        const uint32_t end = !CUT ? PK / 4 : min(PK / 4, 2 * ((k_end - k0 + 8 * KK - 1) / (8 * KK)));
 #pragma unroll 2
         for (uint32_t q = 0; q < end; ++q) {
             float av[NC][4], bv[4];
@@ -368,7 +367,7 @@ __global__ void __launch_bounds__(kT, 4) k_matmul(MatmulArgs g) {
     }
 }
 
-template <bool BT, uint32_t BTYPE, int LOADS, int R, int NC>
+template <bool BT, uint32_t BTYPE, int LOADS, int R, int NC, bool CUT = R == 4>
 void launch_tile(const MatmulArgs& g) {
     constexpr uint32_t WR = R == 1 ? 1 : 2, TM = 16 * NC * WR, TN = 16 * R * (4 / WR);
     dim3 grid((g.p.n + TN - 1) / TN, g.p.batches, (g.p.m + TM - 1) / TM);
@@ -379,7 +378,7 @@ void launch_tile(const MatmulArgs& g) {
         grid.x = rows == 1 ? visible_tiles(g.p, 0, TM, TN) : 2 * visible_tiles(g.p, rows / 2, TM, TN) + 1;
         grid.z = (rows + 1) / 2;
     }
-    hipLaunchKernelGGL((k_matmul<BT, BTYPE, R, NC, LOADS>), grid, dim3(kT), 0, vkml::abi::stream(), g);
+    hipLaunchKernelGGL((k_matmul<BT, BTYPE, R, NC, LOADS, CUT>), grid, dim3(kT), 0, vkml::abi::stream(), g);
 }
 
 template <bool BT, uint32_t BTYPE, int LOADS>
@@ -387,6 +386,9 @@ void launch(const MatmulArgs& g) {
     const WaveTile tile = wave_tile(g.p);
     if constexpr (BTYPE != VKML_Q4_K) {
         if (tile.r == 4) return launch_tile<BT, BTYPE, LOADS, 4, 2>(g);
+    }
+    if constexpr (BT && BTYPE <= VKML_BF16) {
+        if (tile.r == 2 && cut_last_chunk(g.p)) return tile.nc == 2 ? launch_tile<BT, BTYPE, LOADS, 2, 2, true>(g) : launch_tile<BT, BTYPE, LOADS, 2, 1, true>(g);
     }
     if (tile.r == 2) tile.nc == 2 ? launch_tile<BT, BTYPE, LOADS, 2, 2>(g) : launch_tile<BT, BTYPE, LOADS, 2, 1>(g);
     else launch_tile<BT, BTYPE, LOADS, 1, 1>(g);

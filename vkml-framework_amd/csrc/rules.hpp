@@ -63,4 +63,18 @@ inline WaveTile wave_tile(const vkml_matmul_params& p) {
     return {1, 1};
 }
 
+// Whether a 32- or 16-row by 32 tile leaves out the last chunk's k's past the
+// sums (chunks of 32 k's): short sums of a transposed float b that end in a
+// chunk's first half, as the scores of heads of 80. It is a loop of other than
+// constant length, which costs whole chunks (us without and with it, 32 x 32
+// tiles: scores of 2048 queries by 4096 keys, 8 heads of 80, 180, 162; of 72
+// 180, 162; of 128 229, 236; 900 x 8192 x 2048 570, 590; 2048 queries by 4096
+// keys' probs v, 32 heads of 128 in 16 x 32 tiles, 907, 945). The 32 x 64 tile
+// always does (an f32 b's probs v of 1000 queries by 2001 keys 334, 285: it
+// spills fewer registers so; 8192 columns of 2048 k's within 2% either way),
+// the 16 x 16 tile, a chain of chunks that it makes 4 to 10% longer, never.
+inline bool cut_last_chunk(const vkml_matmul_params& p) {
+    return p.b_transposed && p.b_type <= VKML_BF16 && p.k <= 256 && (p.k - 1) % 32 < 16;
+}
+
 }  // namespace vkml::rules
