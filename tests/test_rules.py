@@ -79,3 +79,27 @@ def test_short_sums_that_end_in_a_chunks_first_half_are_cut(rules):
     assert all(cut(k, b) for k in (1, 16, 72, 80, 144, 240) for b in (H.F32, H.F16, H.BF16))
     assert not any(cut(k) for k in (17, 32, 64, 96, 120, 128, 256, 272, 2064))  # (whole chunks and long sums lose by it)
     assert not cut(80, t=0)
+
+
+# us of probs v (f16, heads, queries, first query's position, head_dim)
+PROBS_V_TILES = [
+    (8, 1000, 0, 80, (118, 67.6, 44, 28.5)),
+    (8, 2048, 2048, 128, (476, 295, 268, 251)),
+    (32, 512, 0, 64, (62.5, 35.8, 23.7, 16.1)),
+    (32, 1000, 0, 64, (130, 73, 51.1, 45.6)),
+    (32, 300, 0, 128, (38.5, 23.3, 15.9, 12.9)),
+    (32, 512, 2000, 128, (294, 202, 194, 190)),
+    (32, 2048, 2048, 128, (963, 884, 946, 1010)),
+    (32, 2048, 0, 128, (368, 307, 321, 349)),
+    (32, 1000, 3000, 64, (574, 313, 302, 298)),
+    (64, 2048, 2048, 64, (1340, 936, 1010, 1080)),
+    (64, 1000, 0, 128, (180, 156, 161, 174)),
+    (40, 1700, 0, 128, (316, 273, 286, 302)),
+]
+
+
+@pytest.mark.parametrize("heads,rows,first,hd,us", PROBS_V_TILES)
+def test_masked_probs_v_takes_a_tile_within_5_percent_of_the_fastest(rules, heads, rows, first, hd, us):
+    p = _matmul(rows, hd, rows + first, H.F16, 0, stride=hd * (rows + first), batches=heads, causal=1, offset=first)
+    picked = (42, 22, 21, 11).index(rules.wave_tile_c(C.byref(p)))
+    assert us[picked] <= 1.05 * min(us)

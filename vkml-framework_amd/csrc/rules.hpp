@@ -38,8 +38,8 @@ struct WaveTile {
 
 // The larger a tile, the fewer operands it stages; the smaller, the more
 // waves and the less padding. The lines are at the waves with work that a
-// tile gives; under a causal mask the part of the keys that the average query
-// sees. Measured (us; wave tiles of 32 x 64, 32 x 32, 16 x 32 and 16 x 16):
+// tile gives: of masked scores the part of the keys that the average query
+// sees (of probs v a mask shortens the sums and leaves every tile). Measured (us; wave tiles of 32 x 64, 32 x 32, 16 x 32 and 16 x 16):
 // scores of 2048 queries by 4096 keys, 32 heads of 128, 996, 1015, 1107, 1249;
 // 8192 x 8192 x 128 295, 298, 329, 376; 2048 x 8192 x 2048 1111, 1095, 1155,
 // 1275; probs v at those 2048 queries 952, 909, 942, 1014; 900 x 8192 x 2048
@@ -52,7 +52,7 @@ struct WaveTile {
 // tile, whose headers take the registers that its loads would be in flight in,
 // loses everywhere (2048 x 14336 x 4096 4244 against 4109).
 inline WaveTile wave_tile(const vkml_matmul_params& p) {
-    const double seen = p.causal ? (p.causal_offset + 0.5 * p.m) / (p.causal_offset + 1.0 * p.m) : 1.0;
+    const double seen = p.causal && p.b_transposed ? (p.causal_offset + 0.5 * p.m) / (p.causal_offset + 1.0 * p.m) : 1.0;
     const auto waves = [&](uint64_t r, uint64_t nc) {
         return seen * static_cast<double>((p.m + 16 * nc - 1) / (16 * nc) * ((p.n + 16 * r - 1) / (16 * r)) * p.batches);
     };
