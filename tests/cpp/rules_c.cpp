@@ -9,3 +9,5 @@ extern "C" int float_loads_c(const vkml_matmul_params* p, uint64_t a, uint64_t b
 extern "C" int wave_tile_c(const vkml_matmul_params* p) { return 10 * wave_tile(*p).r + wave_tile(*p).nc; }
 
 extern "C" int cut_last_chunk_c(const vkml_matmul_params* p) { return cut_last_chunk(*p); }
+
+extern "C" uint32_t rows_chunk_c(uint32_t k) { return rows_chunk(k); }

@@ -1254,11 +1254,12 @@ def test_matmul_vec4_and_scalar_loads_agree(bt):
 
 
 @pytest.mark.parametrize("fmt", [H.Q8_0, H.Q4_0, H.Q4_1, H.Q4_K])
-@pytest.mark.parametrize("n,k", [(1, 256), (9, 512), (37, 1792), (16, 2048), (50, 2304), (25, 4096), (21, 96)])
+@pytest.mark.parametrize("n,k", [(1, 256), (9, 512), (37, 1792), (16, 2048), (50, 2304), (25, 4096), (21, 96), (41, 32), (17, 544),
+                                 (33, 768), (8, 800), (19, 1024), (30, 1056)])
 def test_gemv_dot_two_to_eight_rows_bit_exact(fmt, n, k):
-    """The rows kernel's chunks of four rounds (2048 values): whole, a part of
-    one, several and a remainder, for every number of rows, in the oracle's
-    order bit for bit."""
+    """The rows kernel's chunks of four rounds (2048 values), of two (rows of
+    up to 1024) and of one (of up to 768): whole, a part of one, several and a
+    remainder, for every number of rows, in the oracle's order bit for bit."""
     if fmt == H.Q4_K and k % 256:
         k = 256 * (k // 256 + 1)
     v, s, quant, words, scales = weights(fmt, n, k, n + k)

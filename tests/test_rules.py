@@ -103,3 +103,10 @@ def test_masked_probs_v_takes_a_tile_within_5_percent_of_the_fastest(rules, head
     p = _matmul(rows, hd, rows + first, H.F16, 0, stride=hd * (rows + first), batches=heads, causal=1, offset=first)
     picked = (42, 22, 21, 11).index(rules.wave_tile_c(C.byref(p)))
     assert us[picked] <= 1.05 * min(us)
+
+
+# times as fast as the kernel that staged nothing, with chunks of four rounds, two, one (30000 outputs, 2 to 8 rows)
+@pytest.mark.parametrize("k,speed", [(32, (0.79, 1.01, 1.21)), (256, (0.76, 0.99, 1.21)), (512, (0.79, 1.04, 1.24)), (768, (0.93, 1.19, 1.28)),
+                                     (1024, (1.03, 1.32, 1.34)), (1536, (1.18, 1.23, 1.35)), (2048, (1.27, 1.31, 1.34))])
+def test_several_row_gemv_loses_nothing_at_short_rows(rules, k, speed):
+    assert speed[(4, 2, 1).index(rules.rows_chunk_c(k))] > 1

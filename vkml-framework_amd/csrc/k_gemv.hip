@@ -11,6 +11,7 @@
 #include "device.hpp"
 #include "gemv.hpp"
 #include "internal.hpp"
+#include "rules.hpp"
 
 using namespace vkml::dev;
 using namespace vkml::gemv;
@@ -166,8 +167,8 @@ int check_dot_params(const vkml_gemv_dot_params* p, const char* what, bool any_k
 // its M rows in one dispatch): each round of a weight row is loaded and
 // unpacked once and applied to every activation row, each row with its own
 // accumulators in the single-row kernel's order (the same lanes, terms and
-// halving tree). LPR lanes an output row. K runs in chunks of four rounds:
-// the workgroup stages the chunk's codes, code sums and scales of every
+// halving tree). LPR lanes an output row. K runs in chunks of CR rounds (four,
+// fewer for short rows): the workgroup stages the chunk's codes, code sums and scales of every
 // activation row in LDS, and the next chunk's weights and activations are in
 // flight meanwhile. At two rows bound by reading the weights; each further
 // row adds ten VALU operations and 24 bytes from LDS a half-block and lane,
@@ -177,10 +178,10 @@ int check_dot_params(const vkml_gemv_dot_params* p, const char* what, bool any_k
 // 28.9, 35.0 -> 11.5, 17.7, 21.0; q8_0 4096 x 14336 22.5, 26.4, 31.1 -> 12.2,
 // 16.5, 19.2; q4_0 14336 x 4096 12.7, 21.9, 30.1 -> 10.0, 16.3, 19.5. (Two
 // weight rows a lane sharing the LDS reads: within 5% either way.)
-template <int FMT, bool F16S, int LPR, bool FULL, int M>
+template <int FMT, bool F16S, int LPR, bool FULL, int M, uint32_t CR>
 __global__ void __launch_bounds__(256) k_gemv_dot_rows(GemvArgs g, uint32_t m) {
     constexpr int NS = Plan<FMT, LPR>::NS;
-    constexpr uint32_t kRows = 256 / LPR, CR = 4, H = 32 * CR, NL = M * H / 256;
+    constexpr uint32_t kRows = 256 / LPR, H = 32 * CR, NL = (M * H + 255) / 256;
     __shared__ uint4 s_codes[M][H];
     __shared__ float2 s_ss[M][H];
     const uint32_t t = thread_index(), l = t % LPR, grp = t / LPR;
@@ -195,6 +196,7 @@ __global__ void __launch_bounds__(256) k_gemv_dot_rows(GemvArgs g, uint32_t m) {
 #pragma unroll
         for (uint32_t u = 0; u < NL; ++u) {
             const uint32_t e = t + 256 * u, i = min(e / H, m - 1), hb = min(32 * r0 + e % H, halves - 1);
+            if (M * H % 256 != 0 && e >= M * H) break;
             codes[u] = ldg(g.a_values + static_cast<uint64_t>(i) * halves + hb);
             scale[u] = ldg(g.a_scales + static_cast<uint64_t>(i) * (K / 32) + hb / 2);
         }
@@ -216,6 +218,7 @@ __global__ void __launch_bounds__(256) k_gemv_dot_rows(GemvArgs g, uint32_t m) {
 #pragma unroll
         for (uint32_t u = 0; u < NL; ++u) {
             const uint32_t e = t + 256 * u;
+            if (M * H % 256 != 0 && e >= M * H) break;
             s_codes[e / H][e % H] = codes[u];
             s_ss[e / H][e % H] = make_float2(static_cast<float>(byte_sum(codes[u])), scale[u]);
         }
@@ -276,11 +279,19 @@ int launch_rows(const GemvArgs& g, uint32_t m) {
     const dim3 grid((g.n + 256 / LPR - 1) / (256 / LPR));
     vkml::abi::ProfileScope prof("gemv_dot");
     const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, vkml::abi::stream(), g, m); };
-    const bool full = g.k % 512 == 0;
-    if (m <= 2) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 2>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 2>);
-    else if (m <= 4) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 4>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 4>);
-    else if (m <= 6) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 6>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 6>);
-    else full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 8>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 8>);
+    const auto chunk = [&](auto cr) {
+        constexpr uint32_t CR = decltype(cr)::value;
+        const bool full = g.k % 512 == 0;
+        if (m <= 2) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 2, CR>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 2, CR>);
+        else if (m <= 4) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 4, CR>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 4, CR>);
+        else if (m <= 6) full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 6, CR>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 6, CR>);
+        else full ? go(k_gemv_dot_rows<FMT, F16S, LPR, true, 8, CR>) : go(k_gemv_dot_rows<FMT, F16S, LPR, false, 8, CR>);
+    };
+    switch (vkml::rules::rows_chunk(g.k)) {
+        case 1: chunk(std::integral_constant<uint32_t, 1>()); break;
+        case 2: chunk(std::integral_constant<uint32_t, 2>()); break;
+        default: chunk(std::integral_constant<uint32_t, 4>()); break;
+    }
     return vkml::abi::check_launch("gemv_dot");
 }
 

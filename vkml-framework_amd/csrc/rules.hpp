@@ -77,4 +77,16 @@ inline bool cut_last_chunk(const vkml_matmul_params& p) {
     return p.b_transposed && p.b_type <= VKML_BF16 && p.k <= 256 && (p.k - 1) % 32 < 16;
 }
 
+// ---------------------------------------------------------------- vkml_gemv_dot
+
+// The rounds of 512 values that the kernel of 2 to 8 activation rows
+// (k_gemv_dot_rows) stages at a time. Rows shorter than a chunk load and stage
+// its other rounds for nothing. Measured (us; four rounds, two, one; the
+// kernel before it, which staged nothing): q4_K, three rows, 30000 x 256 9.8,
+// 6.7, 5.2 (6.0); q8_0, five rows, 30000 x 512 8.5, 6.8, 5.4 (6.4); the mean
+// over the formats and 2 to 8 rows against that kernel at 30000 x 768 0.93,
+// 1.19, 1.28 times as fast, 8192 x 1024 1.05, 1.23, 1.18, 2048 x 1536 1.17,
+// 1.15, 1.15, 2048 x 2048 1.26, 1.25, 1.16.
+inline uint32_t rows_chunk(uint32_t k) { return k <= 768 ? 1 : k <= 1024 ? 2 : 4; }
+
 }  // namespace vkml::rules
