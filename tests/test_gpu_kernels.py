@@ -1291,6 +1291,21 @@ def test_gemv_float_loads_bit_exact(bt, n, k):
             assert np.array_equal(bits(out.download(np.float32, (m, n))), bits(want)), m
 
 
+@pytest.mark.parametrize("bt", [H.F32, H.F16, H.BF16])
+@pytest.mark.parametrize("n,k", [(8192, 4), (8193, 64), (8200, 128), (8192, 132), (8195, 256), (4096, 68), (4097, 192), (3, 200)])
+def test_gemv_float_short_rows_bit_exact(bt, n, k):
+    """Rows of up to 256 values either side of 8192 outputs, from three rows
+    of a on 4096 (one row of b a half wave up to there, several past it), in
+    one step or two."""
+    rng = np.random.default_rng(n * k + bt)
+    dv, _, ot, ob, _ = _float_b(bt, n, k, rng)
+    for m in range(1, 9):
+        a = rng.standard_normal((m, k)).astype(np.float32)
+        out = H.empty(m * n * 4)
+        H.call("vkml_gemv", H.GemvParams(m, n, k, bt, H.F16, 0, 1, 1), p(dev(a)), p(dv), p(out), None)
+        assert np.array_equal(bits(out.download(np.float32, (m, n))), bits(O.gemv_float(ot, a, ob, None, n, k))), m
+
+
 # The wave tiles of k_matmul_f32.hip's rule (32 x 64, 32 x 32, 16 x 32, 16 x
 # 16), each with ragged rows and columns, a K that ends inside a chunk, and
 # rows that are whole vec4s or not.

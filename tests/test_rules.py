@@ -110,3 +110,13 @@ def test_masked_probs_v_takes_a_tile_within_5_percent_of_the_fastest(rules, head
                                      (1024, (1.03, 1.32, 1.34)), (1536, (1.18, 1.23, 1.35)), (2048, (1.27, 1.31, 1.34))])
 def test_several_row_gemv_loses_nothing_at_short_rows(rules, k, speed):
     assert speed[(4, 2, 1).index(rules.rows_chunk_c(k))] > 1
+
+
+# times as fast as the element-wise kernel at k of up to 128: several rows of b a half wave, one
+@pytest.mark.parametrize("m,n,batches,speed", [(1, 1, 1, (0.97, 1.04)), (1, 256, 1, (0.91, 1.06)), (2, 1000, 1, (0.86, 1.16)),
+                                               (2, 4000, 1, (0.96, 1.22)), (5, 40, 8, (0.98, 1.12)), (8, 64000, 1, (1.19, 0.92)), (5, 4000, 32, (1.35, 1.13)),
+                                               (1, 8000, 1, (1.24, 1.32)), (2, 250, 32, (1.16, 1.32)), (3, 4000, 1, (1.15, 1.18)), (3, 8000, 1, (1.29, 1.24)),
+                                               (5, 250, 32, (1.21, 1.17))])
+def test_float_gemv_of_short_rows_loses_nothing(rules, m, n, batches, speed):
+    picked = speed[rules.gemv_row_each_c(m, n, batches)]
+    assert picked > 1 and picked > 0.9 * max(speed)

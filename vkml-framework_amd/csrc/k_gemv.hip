@@ -508,13 +508,25 @@ __global__ void __launch_bounds__(256) k_gemv_float4_rows(const float* a, uint32
     }
 }
 
+// One row of b a half wave, its U steps at once.
+template <int BT, int U, class Go>
+void short_rows(const Go& go, uint32_t m) {
+    if (m == 1) go(k_gemv_float4<BT, 1, 1, U>, 1);
+    else if (m == 2) go(k_gemv_float4<BT, 2, 1, U>, 1);
+    else if (m <= 4) go(k_gemv_float4<BT, 4, 1, U>, 1);
+    else if (m <= 6) go(k_gemv_float4<BT, 6, 1, U>, 1);
+    else go(k_gemv_float4<BT, 8, 1, U>, 1);
+}
+
 template <int BT>
 void launch_float4(const vkml_gemv_params& p, const float* a, const void* b, float* out, uint32_t batches, uint32_t group) {
     const auto go = [&](auto kernel, uint32_t rows) {
         hipLaunchKernelGGL(kernel, dim3((p.n + 8 * rows - 1) / (8 * rows), batches), dim3(256), 0, vkml::abi::stream(), a, p.m, b, out, p.n, p.k,
                            group, static_cast<uint64_t>(p.b_stride));
     };
-    if (p.k <= 256) {
+    if (p.k <= 256 && vkml::rules::gemv_row_each(p.m, p.n, batches)) {
+        p.k <= 128 ? short_rows<BT, 1>(go, p.m) : short_rows<BT, 2>(go, p.m);
+    } else if (p.k <= 256) {
         // One or two steps a row (attention's scores of up to 8 queries):
         // several rows a lane keep as many loads in flight, and a is read
         // from the caches.

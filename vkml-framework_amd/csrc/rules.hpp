@@ -89,4 +89,19 @@ inline bool cut_last_chunk(const vkml_matmul_params& p) {
 // 1.15, 1.15, 2048 x 2048 1.26, 1.25, 1.16.
 inline uint32_t rows_chunk(uint32_t k) { return k <= 768 ? 1 : k <= 1024 ? 2 : 4; }
 
+// ---------------------------------------------------------------- vkml_gemv
+
+// Whether a float GEMV with rows of up to 256 values (k_gemv_float4) takes one
+// row of b a half wave: with few outputs the launch is one wave's chain of
+// loads, sums and tree, which more rows a lane lengthen; with many the loads
+// in flight a lane matter. Measured as times as fast as the element-wise
+// kernel (the mean over the float types and k of 4 to 128; one row a half
+// wave, against four, or two from three rows of a on): one row of a, 1000
+// outputs 1.10, 0.91, 8000 1.32, 1.24, 64000 1.96, 2.26; two, 1000 1.16,
+// 0.86, 8000 1.32, 1.16, 64000 1.76, 1.82; three, 4000 1.18, 1.15, 8000 1.24,
+// 1.29; five, 1000 1.16, 1.01, 4000 1.16, 1.12, 8000 1.17, 1.21, 64000 1.12,
+// 1.37; eight, 1000 1.18, 1.04, 4000 1.19, 1.15, 9600 1.04, 1.17 (f32 rows of
+// 192 and 256 values, 5000 outputs, eight: 4.7 us, 4.4).
+inline bool gemv_row_each(uint32_t m, uint32_t n, uint32_t batches) { return static_cast<uint64_t>(n) * batches <= (m <= 2 ? 8192 : 4096); }
+
 }  // namespace vkml::rules
