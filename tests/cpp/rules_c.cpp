@@ -13,3 +13,5 @@ extern "C" int cut_last_chunk_c(const vkml_matmul_params* p) { return cut_last_c
 extern "C" uint32_t rows_chunk_c(uint32_t k) { return rows_chunk(k); }
 
 extern "C" int gemv_row_each_c(uint32_t m, uint32_t n, uint32_t batches) { return gemv_row_each(m, n, batches); }
+
+extern "C" int gemv_row_cached_c(const vkml_gemv_params* p) { return gemv_row_cached(*p); }

@@ -1306,6 +1306,24 @@ def test_gemv_float_short_rows_bit_exact(bt, n, k):
         assert np.array_equal(bits(out.download(np.float32, (m, n))), bits(O.gemv_float(ot, a, ob, None, n, k))), m
 
 
+@pytest.mark.parametrize("n,k", [(16384, 4096), (16385, 4096), (16381, 4100)])
+def test_gemv_float_f32_past_the_last_level_cache_bit_exact(n, k):
+    """One row of a by an f32 b either side of 2^26 elements (a staged, or
+    read from the caches), and its last rows against the oracle."""
+    rng = np.random.default_rng(n + k)
+    tail = rng.standard_normal((40, k)).astype(np.float32)
+    a = rng.standard_normal((1, k)).astype(np.float32)
+    b = H.empty(n * k * 4)
+    H.call("vkml_fill_u32", p(b), 0x3F800000, n * k)
+    H.call("vkml_memcpy_h2d", C.c_void_p(p(b).value + (n - 40) * k * 4), tail.ctypes.data_as(C.c_void_p), tail.nbytes)
+    out = H.empty(n * 4)
+    H.call("vkml_gemv", H.GemvParams(1, n, k, H.F32, H.F16, 0, 1, 1), p(dev(a)), p(b), p(out), None)
+    got = out.download(np.float32, (1, n))
+    assert np.array_equal(bits(got[:, -40:]), bits(O.gemv_float(O.T_F32, a, tail, None, 40, k)))
+    ones = O.gemv_float(O.T_F32, a, np.ones((1, k), np.float32), None, 1, k)
+    assert np.array_equal(bits(got[:, :-40]), np.broadcast_to(bits(ones), (1, n - 40)))
+
+
 # The wave tiles of k_matmul_f32.hip's rule (32 x 64, 32 x 32, 16 x 32, 16 x
 # 16), each with ragged rows and columns, a K that ends inside a chunk, and
 # rows that are whole vec4s or not.

@@ -120,3 +120,13 @@ def test_several_row_gemv_loses_nothing_at_short_rows(rules, k, speed):
 def test_float_gemv_of_short_rows_loses_nothing(rules, m, n, batches, speed):
     picked = speed[rules.gemv_row_each_c(m, n, batches)]
     assert picked > 1 and picked > 0.9 * max(speed)
+
+
+# us of one row of a by an f32 b from memory: a staged, a from the caches
+@pytest.mark.parametrize("n,k,us", [(12000, 8192, (73.6, 69.2)), (16000, 8192, (93.3, 90.6)), (32000, 4096, (85.7, 84.7)),
+                                    (8192, 8192, (50.6, 52.2)), (32000, 2048, (42.8, 43.9)), (2048, 8192, (16.4, 17.8))])
+def test_one_row_by_a_large_f32_b_takes_the_faster_form(rules, n, k, us):
+    p = H.GemvParams(1, n, k, H.F32, H.F16, 0, 1, 1)
+    assert us[rules.gemv_row_cached_c(C.byref(p))] == min(us)
+    for m, b_type in ((2, H.F32), (1, H.F16), (1, H.BF16)):
+        assert not rules.gemv_row_cached_c(C.byref(H.GemvParams(m, n, k, b_type, H.F16, 0, 1, 1)))

@@ -535,6 +535,8 @@ void launch_float4(const vkml_gemv_params& p, const float* a, const void* b, flo
         else if (p.m <= 4) go(k_gemv_float4<BT, 4, 2, 1>, 2);
         else if (p.m <= 6) go(k_gemv_float4<BT, 6, 2, 1>, 2);
         else go(k_gemv_float4<BT, 8, 2, 1>, 2);
+    } else if (vkml::rules::gemv_row_cached(p)) {
+        if constexpr (BT == VKML_F32) go(k_gemv_float4<BT, 1, 1, 8>, 1);  // a from the caches
     } else if (p.m == 1) go(k_gemv_float4_rows<BT, 1>, 1);
     else if (p.m == 2) go(k_gemv_float4_rows<BT, 2>, 1);
     else if (p.m <= 4) go(k_gemv_float4_rows<BT, 4>, 1);

@@ -104,4 +104,16 @@ inline uint32_t rows_chunk(uint32_t k) { return k <= 768 ? 1 : k <= 1024 ? 2 : 4
 // 192 and 256 values, 5000 outputs, eight: 4.7 us, 4.4).
 inline bool gemv_row_each(uint32_t m, uint32_t n, uint32_t batches) { return static_cast<uint64_t>(n) * batches <= (m <= 2 ? 8192 : 4096); }
 
+// Whether one row of a by an f32 b of long rows reads a from the caches
+// (k_gemv_float4, eight steps at once) instead of staging it
+// (k_gemv_float4_rows). A b past the 256 MiB of the last-level cache comes
+// from memory at its rate, and the staging's barriers cost more than its reads
+// save. Measured (us; cached, staged; the element-wise kernel): 12000 x 8192
+// 69.2, 73.6 (68.9); 16000 x 8192 90.6, 93.3 (88.9); 32000 x 4096 84.7, 85.7
+// (89.6); up to that size 8192 x 8192 52.2, 50.6 (54.2); 32000 x 2048 43.9,
+// 42.8 (46.6).
+inline bool gemv_row_cached(const vkml_gemv_params& p) {
+    return p.b_type == VKML_F32 && p.m == 1 && p.k >= 4096 && static_cast<uint64_t>(p.n) * p.k > (1u << 26);
+}
+
 }  // namespace vkml::rules
