@@ -15,3 +15,5 @@ extern "C" uint32_t rows_chunk_c(uint32_t k) { return rows_chunk(k); }
 extern "C" int gemv_row_each_c(uint32_t m, uint32_t n, uint32_t batches) { return gemv_row_each(m, n, batches); }
 
 extern "C" int gemv_row_cached_c(const vkml_gemv_params* p) { return gemv_row_cached(*p); }
+
+extern "C" int dot_tail_c(int rt, int ct, uint32_t k) { return dot_tail(rt, ct, k); }

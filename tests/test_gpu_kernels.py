@@ -299,6 +299,27 @@ def test_matmul_dot_tiles_bit_exact(fmt, f16, m, n, k):
     assert np.array_equal(bits(got[rows]), bits(O.matmul_dot(quant, aw, asc, len(rows), words, scales, n, k)))
 
 
+@pytest.mark.parametrize("fmt,f16", [(H.Q8_0, True), (H.Q4_0, False), (H.Q4_1, True), (H.Q4_1, False)])
+@pytest.mark.parametrize("m,n", [(17, 70), (300, 5600), (1100, 3900)])
+def test_matmul_dot_every_length_of_the_last_chunk_bit_exact(fmt, f16, m, n):
+    """K of one and of two chunks whose last has one to eight blocks, in each
+    tile that cuts or masks it, with infinite and NaN scales past K (the next
+    rows'), which no term may reach."""
+    for blocks in (1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 13, 15, 33, 38):
+        k = 32 * blocks
+        v, s, quant, words, scales = weights(fmt, n, k, blocks, f16_scales=f16)
+        a, aw, asc = activation(k, blocks, m)
+        past = np.array([np.inf, np.nan] * 4, np.float32)
+        sc = dev(np.concatenate([np.ascontiguousarray(scales).ravel(), past.astype(np.float16).view(np.uint16) if f16 else past]))
+        act = dev(np.concatenate([np.ascontiguousarray(asc, dtype=np.float32).ravel(), past]))
+        out = H.empty(m * n * 4)
+        H.call("vkml_matmul_dot", H.GemvDotParams(m, n, k, fmt, H.F16 if f16 else H.F32), p(dev(aw)), p(v), p(out), p(sc), p(act))
+        got = out.download(np.float32, (m, n))
+        rows = np.unique(np.concatenate([np.arange(4), np.arange(m - 4, m)]))
+        sub_w, sub_s = np.ascontiguousarray(aw.reshape(m, -1)[rows]), np.ascontiguousarray(asc.reshape(m, -1)[rows])
+        assert np.array_equal(bits(got[rows]), bits(O.matmul_dot(quant, sub_w, sub_s, len(rows), words, scales, n, k))), blocks
+
+
 @pytest.mark.parametrize("fmt", [H.Q8_0, H.Q4_K])
 def test_gemv_dot_add_and_swiglu(fmt):
     n, k = 1024, 4096

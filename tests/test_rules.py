@@ -130,3 +130,11 @@ def test_one_row_by_a_large_f32_b_takes_the_faster_form(rules, n, k, us):
     assert us[rules.gemv_row_cached_c(C.byref(p))] == min(us)
     for m, b_type in ((2, H.F32), (1, H.F16), (1, H.BF16)):
         assert not rules.gemv_row_cached_c(C.byref(H.GemvParams(m, n, k, b_type, H.F16, 0, 1, 1)))
+
+
+# (wave tile, k, us of the last chunk with all its blocks, cut)
+@pytest.mark.parametrize("rt,ct,k,masked,cut", [(2, 2, 32, 5.7, 4.4), (2, 2, 128, 5.7, 5.0), (2, 2, 224, 5.8, 5.7), (1, 1, 32, 3.1, 2.9), (1, 1, 224, 3.13, 3.3),
+                                                (1, 1, 2080, 10.9, 11.3)])
+def test_last_chunk_of_matmul_dot(rules, rt, ct, k, masked, cut):
+    assert rules.dot_tail_c(rt, ct, k) == (2 if cut < masked else 1)
+    assert all(rules.dot_tail_c(rt, ct, whole) == 0 for whole in (256, 512, 4096))

@@ -43,8 +43,10 @@
 #include "../../include/vkml_hip.h"
 #include "device.hpp"
 #include "internal.hpp"
+#include "rules.hpp"
 
 using namespace vkml::dev;
+using namespace vkml::rules;
 
 namespace {
 
@@ -135,7 +137,6 @@ template <int FMT, bool F16S, int RT, int CT>
 struct StagedChunk {
     static constexpr bool kOffset = FMT == VKML_Q4_1 || FMT == VKML_Q4_K;
     static constexpr uint32_t TM = 16 * RT, TN = 64 * CT;     // the tile
-    static constexpr bool kMask = RT * CT != 8;               // blocks past K are computed, as zeros (the largest tile stops at K)
     static constexpr uint32_t kABlocks = RT >= 2 ? RT / 2 : 1;  // a staging thread's A blocks (of one row)
     static constexpr uint32_t kAThreads = TM * kChunk / kABlocks;  // threads that stage A
     static constexpr uint32_t kBBytes = FMT == VKML_Q8_0 ? 256 : 128;  // a column's bytes a chunk
@@ -342,7 +343,7 @@ __device__ __forceinline__ void staged_load(const MatmulDotArgs& p, uint32_t t, 
     }
 }
 
-template <int FMT, bool F16S, int RT, int CT>
+template <int FMT, bool F16S, int RT, int CT, bool MASK>
 __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT, CT>& r, uint32_t t, uint32_t left, StagedLds<FMT, F16S, RT, CT>& l) {
     using S = StagedChunk<FMT, F16S, RT, CT>;
     constexpr bool kOffset = S::kOffset;
@@ -355,12 +356,12 @@ __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT, CT
 #pragma unroll
         for (uint32_t h = 0; h < AB; ++h) {
             const uint32_t b = AB * (t % kPerRow) + h;
-            // Blocks past K (the last chunk of a K of other than whole chunks)
-            // re-read its last one with zero scales, offsets and code sums:
-            // their terms are zeros, which change no accumulator (none is ever
-            // -0).
-            l.sa[b][row] = !S::kMask || b < left ? r.sa[h] : 0.0f;
-            if constexpr (kOffset) l.asum[b][row] = !S::kMask || b < left ? static_cast<float>(byte_sum(r.a[2 * h]) + byte_sum(r.a[2 * h + 1])) : 0.0f;
+            // MASK: blocks past K (the last chunk of a K of other than whole
+            // chunks, whose blocks are scaled in groups) re-read its last one
+            // with zero scales, offsets and code sums: their terms are zeros,
+            // which change no accumulator (none is ever -0).
+            l.sa[b][row] = !MASK || b < left ? r.sa[h] : 0.0f;
+            if constexpr (kOffset) l.asum[b][row] = !MASK || b < left ? static_cast<float>(byte_sum(r.a[2 * h]) + byte_sum(r.a[2 * h + 1])) : 0.0f;
         }
     }
 #pragma unroll
@@ -376,8 +377,8 @@ __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT, CT
             for (uint32_t b = 0; b < 4; ++b) {
                 float sv = r.s[u][b], ov = r.o[u][b];
                 if constexpr (FMT == VKML_Q4_K) q4k_block_scale(r.header[u], b0 + b, sv, ov);
-                l.sb[b0 + b][cl] = !S::kMask || b0 + b < left ? sv : 0.0f;
-                if constexpr (kOffset) l.ob[b0 + b][cl] = !S::kMask || b0 + b < left ? ov : 0.0f;
+                l.sb[b0 + b][cl] = !MASK || b0 + b < left ? sv : 0.0f;
+                if constexpr (kOffset) l.ob[b0 + b][cl] = !MASK || b0 + b < left ? ov : 0.0f;
             }
         }
     }
@@ -411,11 +412,16 @@ __device__ __forceinline__ long staged_b(const StagedLds<FMT, F16S, RT, CT>& l, 
     return static_cast<long>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-template <int FMT, bool F16S, int RT, int CT>
+// TAIL: what the last chunk of K does (rules.hpp).
+template <int FMT, bool F16S, int RT, int CT, int TAIL>
 __global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulDotArgs p) {
     using S = StagedChunk<FMT, F16S, RT, CT>;
     constexpr bool kOffset = S::kOffset;
     constexpr int G = RT * CT >= 4 ? 1 : 4 / (RT * CT);  // blocks whose scaling runs together
+    // (q4_K's K is whole chunks; its tiles with the masks left out are 2 to 7%
+    // slower, as the compiler then orders their staging: 512 x 4096 x 4096
+    // 49.6, 52.0 us)
+    constexpr bool kMask = FMT == VKML_Q4_K ? RT * CT != 8 : TAIL == kMaskedTail || (TAIL == kCutTail && G > 1);
     __shared__ StagedLds<FMT, F16S, RT, CT> l;
     const uint32_t t = thread_index(), lane = t % kWave, wave = t / kWave;
     const uint32_t g = lane / 16, li = lane % 16;
@@ -460,13 +466,15 @@ __global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulD
     staged_load<FMT, F16S, RT, CT>(p, t, 0, row0, col0, next);
     for (uint32_t c0 = 0; c0 < blocks; c0 += kChunk) {
         __syncthreads();  // the last chunk's readers are done
-        staged_store<FMT, F16S, RT, CT>(next, t, blocks - c0, l);
+        staged_store<FMT, F16S, RT, CT, kMask>(next, t, blocks - c0, l);
         __syncthreads();
         if (c0 + kChunk < blocks) staged_load<FMT, F16S, RT, CT>(p, t, c0 + kChunk, row0, col0, next);  // in flight meanwhile
 #pragma unroll
         for (uint32_t b = 0; b < kChunk; b += G) {
+            // (in the largest tile this also keeps the next block's reads, and
+            // their registers, out of this one)
+            if (TAIL == kCutTail && c0 + b >= blocks) break;
             if constexpr (RT * CT == 8) {
-                if (c0 + b >= blocks) break;  // (keeps the next block's reads, and their registers, out of this one)
                 v4i d[RT][CT];
                 sums(b, d);
                 add_large<FMT, F16S, RT, CT>(d, l, b, wave, lane, acc);
@@ -498,7 +506,18 @@ __global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulD
 template <int FMT, bool F16S, int RT, int CT>
 void launch_tile(const MatmulDotArgs& p) {
     const dim3 grid((p.n + 64 * CT - 1) / (64 * CT), (p.m + 16 * RT - 1) / (16 * RT));
-    hipLaunchKernelGGL((k_matmul_dot<FMT, F16S, RT, CT>), grid, dim3(kT), 0, vkml::abi::stream(), p);
+    const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kT), 0, vkml::abi::stream(), p); };
+    const DotTail tail = dot_tail(RT, CT, p.k);
+    if constexpr (RT * CT == 8) {
+        go(k_matmul_dot<FMT, F16S, RT, CT, kCutTail>);
+    } else if constexpr (FMT == VKML_Q4_K) {  // (its K is whole chunks)
+        go(k_matmul_dot<FMT, F16S, RT, CT, kWholeTail>);
+    } else {
+        if constexpr (RT * CT == 1) {
+            if (tail == kMaskedTail) return go(k_matmul_dot<FMT, F16S, RT, CT, kMaskedTail>);
+        }
+        tail == kWholeTail ? go(k_matmul_dot<FMT, F16S, RT, CT, kWholeTail>) : go(k_matmul_dot<FMT, F16S, RT, CT, kCutTail>);
+    }
 }
 
 // Tiles of 64 x 128, 32 x 128, 16 x 128 and 16 x 64 outputs, the larger while

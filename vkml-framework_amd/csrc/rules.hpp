@@ -77,6 +77,24 @@ inline bool cut_last_chunk(const vkml_matmul_params& p) {
     return p.b_transposed && p.b_type <= VKML_BF16 && p.k <= 256 && (p.k - 1) % 32 < 16;
 }
 
+// ---------------------------------------------------------------- vkml_matmul_dot
+
+// The last chunk of K, 8 blocks of 32, in k_matmul_dot (k_matmul.hip): whole
+// (no masks, no branch); all its blocks, those past K as zeros; or only the
+// groups of blocks (one, two or, in the 16 x 64 tile, four) that hold some,
+// at a branch a group in every chunk.
+enum DotTail { kWholeTail = 0, kMaskedTail = 1, kCutTail = 2 };
+
+// rt, ct: a wave's tile, 16 rt rows by 16 ct columns. Measured (us; masked,
+// cut): q8_0 300 x 4096 (32 x 128 tiles), K of 32 5.7, 4.4; 128 5.7, 5.0; 224
+// 5.8, 5.7; 2080 equal. In the 16 x 64 tile the cut saves half a chunk or
+// nothing, and its branch costs 5%: q8_0 64 x 4096, K of 32 3.1, 2.9; q4_1 64 x
+// 4096, 224 3.13, 3.3, 2080 10.9, 11.3.
+inline DotTail dot_tail(int rt, int ct, uint32_t k) {
+    if (k % 256 == 0) return kWholeTail;
+    return rt * ct > 1 || (k % 256 <= 128 && k <= 1024) ? kCutTail : kMaskedTail;
+}
+
 // ---------------------------------------------------------------- vkml_gemv_dot
 
 // The rounds of 512 values that the kernel of 2 to 8 activation rows
