@@ -17,3 +17,9 @@ extern "C" int gemv_row_each_c(uint32_t m, uint32_t n, uint32_t batches) { retur
 extern "C" int gemv_row_cached_c(const vkml_gemv_params* p) { return gemv_row_cached(*p); }
 
 extern "C" int dot_tail_c(int rt, int ct, uint32_t k) { return dot_tail(rt, ct, k); }
+
+// 10 rt + ct
+extern "C" int dot_tile_c(uint32_t b_type, int f16_scales, uint32_t m, uint32_t n) {
+    const DotTile t = dot_tile(b_type, f16_scales != 0, m, n);
+    return 10 * t.rt + t.ct;
+}

@@ -283,10 +283,11 @@ def test_matmul_dot_bit_exact(fmt, f16, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(9, 70, 96), (33, 65, 288), (17, 1000, 2336), (150, 2500, 544), (119, 8200, 544), (139, 8200, 32),
                                    (530, 3872, 800), (2050, 8200, 288)])
 def test_matmul_dot_tiles_bit_exact(fmt, f16, m, n, k):
-    # The four tiles of launch()'s rule (16 x 64 in the first four, 16 x 128
-    # and 32 x 128 with 1028 and 1285 or more waves of 32 x 32, 64 x 128),
-    # ragged both ways, with a K that ends inside a chunk of 8 blocks and of
-    # one, two and several chunks.
+    # The tiles of dot_tile's rule (16 x 64 in the first four; 16 x 128 with
+    # 1028 waves of 32 x 32 for q4_K and q4_1 with f32 scales; 32 x 128 with
+    # 1285 for q8_0 and 2057 for all; 64 x 128 for q4_0 and q4_K), ragged both
+    # ways, with a K that ends inside a chunk of 8 blocks and of one, two and
+    # several chunks.
     if fmt == H.Q4_K:
         k = 256 * (k // 256 + 1)
     v, s, quant, words, scales = weights(fmt, n, k, m + n, f16_scales=f16)
@@ -300,7 +301,7 @@ def test_matmul_dot_tiles_bit_exact(fmt, f16, m, n, k):
 
 
 @pytest.mark.parametrize("fmt,f16", [(H.Q8_0, True), (H.Q4_0, False), (H.Q4_1, True), (H.Q4_1, False)])
-@pytest.mark.parametrize("m,n", [(17, 70), (300, 5600), (1100, 3900)])
+@pytest.mark.parametrize("m,n", [(17, 70), (300, 5600), (300, 3100)])
 def test_matmul_dot_every_length_of_the_last_chunk_bit_exact(fmt, f16, m, n):
     """K of one and of two chunks whose last has one to eight blocks, in each
     tile that cuts or masks it, with infinite and NaN scales past K (the next

@@ -520,23 +520,16 @@ void launch_tile(const MatmulDotArgs& p) {
     }
 }
 
-// Tiles of 64 x 128, 32 x 128, 16 x 128 and 16 x 64 outputs, the larger while
-// the SIMDs still get waves enough. Measured (us; those four): q4_K 4096 x
-// 14336 x 4096 999, 1054, -, -; 4096 x 4096 x 14336 1003, 1049, -, -; 512 x
-// 14336 x 4096 169, 148, 179, 231; 512 x 4096 x 14336 245, 166, 183, 236; 300
-// x 8192 x 2048 47, 37, 36, 45; 300 x 3072 x 2048 37, 23, 18, 21; 300 x 2048 x
-// 8192 139, 80, 62, 57; 37 x 4096 x 14336 237, 139, 87, 66; q8_0 131 x 8192 x
-// 2048 37, 28, 30, 31; 131 x 2048 x 8192 124, 77, 62, 44. (16 x 256 and 32 x
-// 256 tiles lost throughout: 213 to 241 VGPRs. A second chunk in flight in
-// registers gained up to 4% at q4_K products of few workgroups and lost 15 to
-// 20% on the other formats, whose scales take more registers.)
 template <int FMT, bool F16S>
 void launch(const MatmulDotArgs& p) {
-    const auto waves = [&](uint64_t rt, uint64_t ct) { return ((p.m + 16 * rt - 1) / (16 * rt)) * ((p.n + 16 * ct - 1) / (16 * ct)); };
-    if (waves(4, 2) >= 8192) launch_tile<FMT, F16S, 4, 2>(p);
-    else if (waves(2, 2) >= 1280) launch_tile<FMT, F16S, 2, 2>(p);
-    else if (waves(2, 2) >= 900) launch_tile<FMT, F16S, 1, 2>(p);
-    else launch_tile<FMT, F16S, 1, 1>(p);
+    const DotTile tile = dot_tile(FMT, F16S, p.m, p.n);
+    if constexpr (dot_has_64_rows(FMT)) {
+        if (tile.rt == 4) return launch_tile<FMT, F16S, 4, 2>(p);
+    }
+    if constexpr (dot_has_16x128(FMT, F16S)) {
+        if (tile.rt == 1 && tile.ct == 2) return launch_tile<FMT, F16S, 1, 2>(p);
+    }
+    tile.rt == 2 ? launch_tile<FMT, F16S, 2, 2>(p) : launch_tile<FMT, F16S, 1, 1>(p);
 }
 
 int matmul_dot_common(const char* what, const vkml_gemv_dot_params* p, const void* a_values, const void* b_values, float* out,

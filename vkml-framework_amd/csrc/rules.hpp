@@ -79,7 +79,46 @@ inline bool cut_last_chunk(const vkml_matmul_params& p) {
 
 // ---------------------------------------------------------------- vkml_matmul_dot
 
-// The last chunk of K, 8 blocks of 32, in k_matmul_dot (k_matmul.hip): whole
+// A wave's tile in k_matmul_dot (k_matmul.hip): 16 rt rows by 16 ct columns;
+// four of them side by side are a workgroup's.
+struct DotTile {
+    int rt, ct;
+};
+
+// Tiles of 64 x 128, 32 x 128, 16 x 128 and 16 x 64 outputs: a larger one
+// stages less for each output and scales more of them at a time, a smaller one
+// gives the SIMDs more waves, and the formats differ in the registers that
+// their scales take. The lines, by waves of a 64 x 32 or 32 x 32 tile (1024
+// SIMDs), are where the times cross over. Measured (us; those four):
+// q4_K: 512 x 2048 x 2048 (1024 waves) 36, 22, 17.9, 19.4; 384 x 4096 x 4096
+// (1536) 68, 50, 42.6, 53; 800 x 2048 x 8192 (1600) 134, 93.4, 114, 114; 512 x
+// 14336 x 4096 158, 134, 173, 215; 1000 x 14336 x 4096 264, 258, 336, 411; 4096
+// x 4096 x 4096 287, 292, 383, 469; 40 and 64 x 14336 x 4096 (896) 29.1 and
+// 36.2 in 16 x 64, 31.9 and 33.2 in 16 x 128.
+// q4_0: 256 x 4096 x 4096 (1024) 69, 43, 37, 31; 300 x 4096 x 4096 (1280) 69,
+// 50, 48, 36; 384 x 4096 x 4096 (1536) 70, 50, 48, 49; 512 x 4096 x 4096 (2048)
+// 71, 52, 57, 58.
+// q8_0: 256 x 4096 x 4096 68, 41, 36, 34; 131 x 8192 x 2048 (1280) 36, 25.4,
+// 26.9, 26.5; 128 x 14336 x 4096 72, 51, 75, 63; 4096 x 4096 x 4096 334, 307,
+// 449, 448; with f32 scales 131 x 8192 x 2048 32, 24.3, 24.3, 21.5.
+// q4_1: 4096 x 4096 x 4096 311, 299, 433, 453; with f32 scales 384 x 4096 x
+// 4096 77, 56, 48, 53; 3000 x 6144 x 4096 422, 386, 456, 567.
+// (16 x 256 and 32 x 256 tiles lost throughout: 213 to 241 VGPRs. A second
+// chunk in flight in registers gained up to 4% at q4_K products of few
+// workgroups and lost 15 to 20% on the other formats, whose scales take more
+// registers.)
+constexpr bool dot_has_64_rows(uint32_t b_type) { return b_type == VKML_Q4_0 || b_type == VKML_Q4_K; }
+constexpr bool dot_has_16x128(uint32_t b_type, bool f16_scales) { return b_type == VKML_Q4_K || (b_type == VKML_Q4_1 && !f16_scales); }
+
+inline DotTile dot_tile(uint32_t b_type, bool f16_scales, uint32_t m, uint32_t n) {
+    const auto waves = [&](uint64_t rt, uint64_t ct) { return ((m + 16 * rt - 1) / (16 * rt)) * ((n + 16 * ct - 1) / (16 * ct)); };
+    if (dot_has_64_rows(b_type) && waves(4, 2) >= 8192) return {4, 2};
+    if (waves(2, 2) >= (b_type == VKML_Q8_0 && f16_scales ? 1280 : 1600)) return {2, 2};
+    if (dot_has_16x128(b_type, f16_scales) && waves(2, 2) >= 900) return {1, 2};
+    return {1, 1};
+}
+
+// The last chunk of K, 8 blocks of 32, in k_matmul_dot: whole
 // (no masks, no branch); all its blocks, those past K as zeros; or only the
 // groups of blocks (one, two or, in the 16 x 64 tile, four) that hold some,
 // at a branch a group in every chunk.
