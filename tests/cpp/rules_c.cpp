@@ -23,3 +23,7 @@ extern "C" int dot_tile_c(uint32_t b_type, int f16_scales, uint32_t m, uint32_t 
     const DotTile t = dot_tile(b_type, f16_scales != 0, m, n);
     return 10 * t.rt + t.ct;
 }
+
+extern "C" int wide_blocks_c(const vkml_attend_prompt_params* p, uint32_t workgroups, uint32_t compute_units) {
+    return wide_blocks(*p, workgroups, compute_units);
+}

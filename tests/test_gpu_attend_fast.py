@@ -237,6 +237,8 @@ PROMPT_SHAPES = [
     # whole number of blocks and one more, tiles that start in a later block
     (8, 2, 64, 0, 64, 64), (8, 2, 64, 1, 64, 70), (32, 8, 128, 0, 192, 192), (8, 2, 128, 3, 190, 200),
     (4, 1, 128, 240, 17, 257), (8, 1, 128, 63, 193, 256), (32, 8, 128, 0, 1024, 1024), (32, 8, 128, 1, 1025, 1030),
+    (8, 2, 128, 0, 33, 40), (8, 2, 128, 31, 65, 96), (8, 2, 64, 40, 57, 100), (8, 2, 128, 0, 129, 129), (8, 2, 64, 0, 129, 130),
+    (32, 8, 128, 0, 1537, 1540), (32, 8, 128, 1025, 1025, 2050),
 ]
 
 

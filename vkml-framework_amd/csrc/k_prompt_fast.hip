@@ -42,6 +42,7 @@
 #include "attend_fast.hpp"
 #include "device.hpp"
 #include "internal.hpp"
+#include "rules.hpp"
 
 using namespace vkml::dev;
 using vkml::attend::kThreads;
@@ -316,20 +317,6 @@ __global__ void __launch_bounds__(kThreads) k_attend_prompt_fast(PromptArgs a) {
     }
 }
 
-// Whether a block is 64 keys instead of 32: half the waits, barriers and
-// maxima a key and more independent matrix instructions between them, against
-// half a block more of masked keys a tile and twice the LDS, which at head_dim
-// 128 leaves two workgroups a compute unit. Measured (us; 32, 64; 32 heads on
-// 8 KV heads; before the matrix instructions were interleaved): head_dim 128, 40 queries 5.6, 6.1; 130 8.8, 9.2; 200 11.7,
-// 11.7; 300 16.0, 14.9; 512 23.7, 21.2; 64 after 1000 keys 43.3, 37.9; 1000
-// after 37 44.7, 41.9; 2048 (four workgroups a compute unit) 90.5, 94.3;
-// head_dim 64, 9 queries 3.6, 4.0; 64 after 64 keys 6.2, 5.7; 300 11.2, 9.9;
-// 1000 29.6, 25.7; 2048 after 2048 keys 147, 140.
-bool wide_blocks(const vkml_attend_prompt_params& p, uint32_t workgroups) {
-    const uint32_t keys = p.first + p.t;
-    return p.head_dim == 64 ? keys > 64 : keys > 192 && workgroups <= 2 * vkml::abi::compute_units();
-}
-
 const char* check_prompt(const vkml_attend_prompt_params* p) {
     if (!p) return "null params";
     if (p->kv_type != VKML_F16) return "caches must be f16";
@@ -358,7 +345,7 @@ int vkml_attend_prompt_fast(const vkml_attend_prompt_params* p, const float* q, 
     const dim3 grid((p->t + kQueries - 1) / kQueries * (p->kv_heads * (a.group / kHeads)));
     vkml::abi::ProfileScope prof("attend_prompt_fast");
     const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, vkml::abi::stream(), a); };
-    const bool wide = wide_blocks(*p, grid.x);
+    const bool wide = vkml::rules::wide_blocks(*p, grid.x, vkml::abi::compute_units());
     if (p->head_dim == 128) wide ? go(k_attend_prompt_fast<128, 64>) : go(k_attend_prompt_fast<128, 32>);
     else wide ? go(k_attend_prompt_fast<64, 64>) : go(k_attend_prompt_fast<64, 32>);
     return vkml::abi::check_launch("attend_prompt_fast");

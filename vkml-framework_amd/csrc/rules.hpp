@@ -173,4 +173,25 @@ inline bool gemv_row_cached(const vkml_gemv_params& p) {
     return p.b_type == VKML_F32 && p.m == 1 && p.k >= 4096 && static_cast<uint64_t>(p.n) * p.k > (1u << 26);
 }
 
+// ---------------------------------------------------------------- vkml_attend_prompt_fast
+
+// Whether k_attend_prompt_fast's blocks are of 64 keys instead of 32: half the
+// waits, barriers and maxima a key and twice the independent matrix
+// instructions between them, against up to half a block of masked keys more,
+// where the keys are few and an odd number of 32s, and, at head_dim 128, LDS
+// that leaves two workgroups a compute unit instead of four. A third round of
+// those pays only where the tiles' lengths differ (the longest start first),
+// as they do from position 0. Measured (us; 32, 64; 32 heads on 8 KV heads):
+// head_dim 128, 9 queries 4.3, 4.9; 40 5.6, 5.8; 64 6.4, 6.0; 90 7.5, 7.8; 128 8.8, 7.9; 150
+// 9.9, 9.7; 192 11.0, 9.9; 300 15.6, 13.7; 64 after 1000 keys 42.2, 34.6; 1000
+// after 37 43.1, 38.3; 1100 (552 workgroups) 46.2, 39.7, after 4000 keys 236,
+// 273; 1500 (752) 61.6, 53.3; 2048 (1024) 88.6, 93.2; head_dim 64, 9 queries
+// 3.4, 3.8; 64 4.56, 4.33; 90 5.36, 5.48; 128 6.2, 5.5; 1000 28.8, 23.1; 2048
+// after 2048 keys 151, 142.
+inline bool wide_blocks(const vkml_attend_prompt_params& p, uint32_t workgroups, uint32_t compute_units) {
+    const uint32_t keys = p.first + p.t;
+    if (keys <= 48 || (keys <= 128 && (keys + 31) / 32 % 2 != 0)) return false;
+    return p.head_dim == 64 || workgroups <= 2 * compute_units || (workgroups <= 3 * compute_units && p.first < p.t);
+}
+
 }  // namespace vkml::rules
