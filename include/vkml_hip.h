@@ -197,9 +197,9 @@ int vkml_dequantize(const vkml_dequantize_params* p, const void* d_values, const
 
 /* The largest k the one-row int8 GEMVs stage in LDS. Above it (any
  * multiple of 32 for q8_0 / q4_0 / q4_1, of 256 for q4_K), vkml_gemv_dot
- * and vkml_gemv_dot_add take the rows kernel, which reads the activation
- * from memory, in the same order; the fused forms (SwiGLU, RMSNorm
- * prologue) take k up to this bound. */
+ * and vkml_gemv_dot_add take the rows kernel, which stages the activation
+ * in chunks, in the same order; the fused forms (SwiGLU, RMSNorm prologue)
+ * take k up to this bound. */
 #define VKML_GEMV_STAGED_MAX_K 32768u
 
 /* shaders/gemv_dot.comp, src/ops/matmul.cpp:225-245: c[m, n] = a_q[m] . b[n]

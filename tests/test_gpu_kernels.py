@@ -1456,6 +1456,53 @@ def test_matmul_quantized_tiles_bit_exact(fmt, f16, m, n, k, shift):
     assert np.array_equal(bits(got[rows]), bits(want))
 
 
+def _same_or_both_nan(got, want):
+    return np.all((bits(got) == bits(want)) | (np.isnan(got) & np.isnan(want)))
+
+
+@pytest.mark.parametrize("transposed", [1, 0])
+@pytest.mark.parametrize("batches,m,n,k", [(32, 530, 2052, 36), (16, 530, 1028, 68), (8, 401, 1004, 100), (1, 17, 70, 33)])
+def test_matmul_infinities_and_nan(transposed, batches, m, n, k):
+    """Infinite and NaN elements of a and b reach the outputs of their own
+    rows and columns alone, as the oracle's (NaN where it has one), in each
+    wave tile: the matrix instruction forms the products of many at once."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((batches, m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k)).astype(np.float32)
+    for z in (0, batches - 1):
+        a[z, 3, k // 2], a[z, 5, 0], a[z, m - 1, k - 1] = np.inf, np.nan, -np.inf
+    b[2, k // 2], b[n - 1, k - 1], b[7, 1] = -np.inf, np.nan, 3e38
+    db = dev(b if transposed else np.ascontiguousarray(b.T))
+    out = H.empty(batches * m * n * 4)
+    H.call("vkml_matmul", H.MatmulParams(m, n, k, 0, batches, batches, transposed, H.F32, H.F16), p(dev(a)), p(db), p(out), None)
+    got = out.download(np.float32, (batches, m, n))
+    rows = [0, 3, 4, 5, 6, m - 2, m - 1]
+    for z in (0, batches - 1):
+        assert _same_or_both_nan(got[z][rows], O.matmul_float(O.T_F32, a[z][rows], b, None, n, k)), z
+
+
+@pytest.mark.parametrize("fmt", [H.Q8_0, H.Q4_0, H.Q4_1])
+@pytest.mark.parametrize("m,n", [(17, 70), (300, 3100), (300, 5600)])
+def test_matmul_dot_infinite_and_nan_scales(fmt, m, n):
+    """An infinite or NaN scale of a row or a column reaches that row's or
+    column's outputs alone, as the oracle's, where the terms of sixteen
+    outputs come from one matrix instruction. (Of q4_1 the offset: its folded
+    scaling makes an infinite f16 scale NaN where the reference has infinity.)"""
+    k = 288
+    v, _, quant, words, scales = weights(fmt, n, k, m + n, f16_scales=True)
+    a, aw, asc = activation(k, m, m)
+    asc = np.ascontiguousarray(asc, dtype=np.float32).reshape(m, -1).copy()
+    asc[3, 1], asc[m - 1, 8] = np.inf, np.nan
+    sc = np.ascontiguousarray(scales).reshape(n, -1).copy()
+    sc[5, 1 if fmt == H.Q4_1 else 0], sc[n - 1, -1] = 0x7C00, 0x7E00  # infinity, NaN
+    out = H.empty(m * n * 4)
+    H.call("vkml_matmul_dot", H.GemvDotParams(m, n, k, fmt, H.F16), p(dev(aw)), p(v), p(out), p(dev(sc)), p(dev(asc)))
+    got = out.download(np.float32, (m, n))
+    rows = [0, 2, 3, 4, 16, m - 2, m - 1]
+    want = O.matmul_dot(quant, np.ascontiguousarray(aw.reshape(m, -1)[rows]), asc[rows], len(rows), words, sc.reshape(np.asarray(scales).shape), n, k)
+    assert _same_or_both_nan(got[rows], want)
+
+
 @pytest.mark.parametrize("rows,first", [(130, 0), (64, 70), (200, 3)])
 def test_matmul_causal_skip_changes_nothing(rows, first):
     """The causal skip: scores on and below the diagonal (row r sees keys

@@ -359,9 +359,11 @@ __global__ void __launch_bounds__(256) k_gemv_float(const float* a, uint32_t m, 
 
 // The same order for a float b whose rows are whole, aligned groups of four
 // (k % 4 == 0): a lane loads a group with one 8- or 16-byte load, U steps of
-// R rows at once, the next batch's loads in flight while this one is summed.
-// For rows of one or two steps (scores of 32 heads of 128 against 4000 keys:
-// two queries 20 -> 11 us, eight 30 -> 23.5).
+// R rows at once, the next batch's loads in flight while this one is summed,
+// a from the caches. For rows of one or two steps (scores of 32 heads of 128
+// against 4000 keys: two queries 20 -> 11 us, eight 30 -> 23.5; a row a half
+// wave where the outputs are few, two rows of a by 1000 x 64 2.4 -> 2.1), and
+// for one row of a by an f32 b past the last-level cache (gemv_row_cached).
 template <int BT>
 using Group4 = std::conditional_t<BT == VKML_F32, uint4, uint2>;
 
@@ -569,7 +571,7 @@ int vkml_gemv_dot_add(const vkml_gemv_dot_params* p, const void* a_values, const
     if (p->n == 0) return VKML_OK;
     VKML_CHECK_ARG(a_values && b_values && out && b_scales && a_scales && residual, "gemv_dot_add: null buffer");
     GemvArgs g{static_cast<const uint4*>(a_values), a_scales, b_values, b_scales, nullptr, nullptr, out, residual, p->n, p->k};
-    if (p->k > kMaxK) return dispatch_rows(p->b_type, p->scale_type, g, 1);  // the activation read from memory
+    if (p->k > kMaxK) return dispatch_rows(p->b_type, p->scale_type, g, 1);  // the activation staged in chunks
     return dispatch_format<kAdd>(p->b_type, p->scale_type, g, "gemv_dot_add");
 }
 

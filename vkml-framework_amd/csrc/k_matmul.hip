@@ -384,7 +384,8 @@ __device__ __forceinline__ void staged_store(const StagedChunk<FMT, F16S, RT, CT
     }
 }
 
-// Column cl's operand for block b of the staged chunk (as b_codes).
+// Column cl's operand for block b of the staged chunk: its 8 codes at values
+// 8 g .. 8 g + 7, as int8 (q4: codes 0 .. 15, or minus 8 for q4_0).
 template <int FMT, bool F16S, int RT, int CT>
 __device__ __forceinline__ long staged_b(const StagedLds<FMT, F16S, RT, CT>& l, uint32_t cl, uint32_t b, uint32_t g) {
     using S = StagedChunk<FMT, F16S, RT, CT>;
