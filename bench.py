@@ -67,11 +67,11 @@ PROMPT = 4096
 # kernel sources it was taken on: its hash is the SHA-256 (first 16 hex
 # digits) of those files, and the line reports no traffic when they have
 # changed since.
-GATE_UP_TRAFFIC = 67_423_679
-GATE_UP_TRAFFIC_SOURCES = "8ab00a5e354809b3"
+GATE_UP_TRAFFIC = 67_446_452
+GATE_UP_TRAFFIC_SOURCES = "8fa86e1feddb6079"
 TRAFFIC_FILES = ("vkml-framework_amd/csrc/gemv.hpp", "vkml-framework_amd/csrc/k_gemv.hip", "vkml-framework_amd/csrc/device.hpp")
-ATTEND_TRAFFIC = 28_559_753
-ATTEND_TRAFFIC_SOURCES = "25b8fc154c973f36"
+ATTEND_TRAFFIC = 28_565_914
+ATTEND_TRAFFIC_SOURCES = "0ba1147ec8bdd50a"
 ATTEND_TRAFFIC_POSITION = 4224  # the launch's shape the figure was taken at (position; 35 chunks, 32 loading early)
 ATTEND_FILES = ("vkml-framework_amd/csrc/k_attend.hip", "vkml-framework_amd/csrc/attend.hpp", "vkml-framework_amd/csrc/gemv.hpp",
                 "vkml-framework_amd/csrc/device.hpp")
