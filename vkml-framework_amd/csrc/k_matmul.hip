@@ -27,17 +27,18 @@
 //
 // What bounds it. The scaling costs 4 operations per output and block (the
 // offset formats' six folded into four, as kSumBiasBits says), which issue at
-// 1.0 (mul, add) to 1.25 ns (fma) a wave64 instruction on a SIMD with two
-// waves or more ready, and the matrix instructions, 7 ns each, hide little of
-// it: 5.7 ns for a lane's output and block, 740 TOP/s, when nothing waits.
-// The large products reach 480 TOP/s, the 512-row ones 360 to 440. One
-// operation in four is an outer product of a row tile's and a column tile's
-// values, which the matrix unit forms for sixteen outputs a lane at once
-// (add_tiles); with the others run sixteen at a time that took 512 x 14336 x
-// 4096 (q4_K) from 156 to 148 us, 512 x 4096 x 14336 181 -> 166, 1000 x 8192
-// x 3072 (q4_1) 143 -> 128. The 16 x 64 tiles replace kernels that loaded
-// operands from memory block by block: 131 x 2048 x 8192 (q8_0) 130 -> 52 us,
-// 37 x 4096 x 14336 145 -> 66, 9 x 4096 x 4096 34 -> 20.
+// about 1.04 ns a wave64 instruction on a SIMD with waves enough, and the int8
+// matrix instructions, 6.8 ns each, run beside them only in part. One operation
+// in four is an outer product of a row tile's and a column tile's values, which
+// the matrix unit forms for sixteen outputs a lane at once, 0.85 ns each
+// (add_tiles): 22.7 ns for a lane's four outputs of a block, 740 TOP/s, when
+// nothing waits and nothing overlaps. The large products reach 480 TOP/s, the
+// 512-row ones 360 to 440: they fill 57 to 80% of their time. Against kernels
+// that formed that product on the VALU, and loaded the operands of small
+// products from memory block by block (us): 512 x 14336 x 4096 (q4_K) 152 ->
+// 141, 512 x 4096 x 14336 179 -> 164, 1000 x 8192 x 3072 (q4_1) 140 -> 121; 131
+// x 2048 x 8192 (q8_0) 116 -> 39, 37 x 4096 x 14336 135 -> 63, 9 x 4096 x 4096
+// 33.5 -> 19.8.
 #include <algorithm>
 
 #include "../../include/vkml_hip.h"

@@ -10,16 +10,23 @@
 // the bits of the VALU's product, subnormals included. (A product of -0
 // comes out +0; no sum that starts at +0 can tell.)
 //
-// What bounds it. The add of every product: a SIMD with two waves or more
-// issues a wave64 add about every 1.0 ns, and the matrix unit, which hardly
-// runs beside the VALU, takes 0.86 ns for a lane's product: 1.8 ns for the
-// two at best, 36 T multiply-accumulates a second over the GPU, of which the
-// large products reach 30. The kernel before it, 4 x 4 outputs a thread with
-// a multiply and an add each, read 512 values from LDS for 1024 products,
-// where a wave here reads 96 for 2048, and reached 20 to 26. Measured before
-// and after (us): probs v of 2048 queries by 4096 keys, 32 heads of 128,
-// 1303 -> 909, its scores 1257 -> 996; 512 queries from position 0 60 -> 27
-// and 46 -> 29; 200 x 8192 x 2048 228 -> 161, 200 x 2048 x 8192 875 -> 216.
+// What bounds it. The add of every product: a SIMD with waves enough issues a
+// wave64 add about every 1.04 ns, and the matrix unit, which does not run
+// beside the VALU, takes 0.85 ns for a lane's product: 1.9 ns for the two at
+// best, 34.6 T multiply-accumulates a second over the GPU (a loop of nothing
+// else reaches 31.5), of which the large products reach 30. The kernel before
+// it, 4 x 4 outputs a thread with a multiply and an add each, read 512 lane
+// values from LDS for a wave's 1024 products, where a wave here reads 192 for
+// 2048, and reached 20 to 26. Measured before and after (us; f16 b): probs v of
+// 2048 queries by 4096 keys, 32 heads of 128, 1287 -> 915, its scores 1152 ->
+// 912; 512 queries from position 0 60 -> 26 and 46 -> 29; 200 x 8192 x 2048
+// 209 -> 154, 200 x 2048 x 8192 863 -> 218. A quantized b's codes are widened
+// when they are staged (q4_K 512 x 4096 x 4096 719 -> 384).
+//
+// Registers. Four waves a SIMD; the element-load forms of an f32 b and three
+// 32-row tiles of quantized ones spill up to nine registers for it. With three
+// waves and none spilled they are equal or up to 3% slower (2000 x 8193 x 1025,
+// f32 b by elements, 694, 704 us).
 //
 // Mapping. A wave computes 16 NC rows by 16 R columns; one instruction's
 // four 16 x 16 blocks are R column blocks by 4 / R consecutive k's, so that
