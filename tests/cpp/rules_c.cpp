@@ -27,3 +27,14 @@ extern "C" int dot_tile_c(uint32_t b_type, int f16_scales, uint32_t m, uint32_t 
 extern "C" int wide_blocks_c(const vkml_attend_prompt_params* p, uint32_t workgroups, uint32_t compute_units) {
     return wide_blocks(*p, workgroups, compute_units);
 }
+
+// The tiles of a launch in the order of its workgroups, 65536 row + col, ~0 for none; the number of workgroups.
+extern "C" uint32_t dot_bands_c(uint32_t rows, uint32_t columns, uint32_t* tiles) {
+    const DotBands b = dot_bands(rows, columns);
+    if (b.width == 0) return 0;
+    for (uint32_t i = 0; i < 8 * b.share; ++i) {
+        uint32_t row, col;
+        tiles[i] = b.tile(i, row, col) ? 65536 * row + col : ~0u;
+    }
+    return 8 * b.share;
+}

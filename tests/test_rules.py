@@ -285,3 +285,21 @@ def test_prompt_attention_takes_the_faster_block(rules, heads, kv_heads, hd, fir
     p = H.AttendPromptParams(heads, kv_heads, hd, first + t, t, first, H.F16, 1.0, 0.0)
     workgroups = -(-t // 16) * kv_heads * max(1, heads // kv_heads // 4)
     assert rules.wide_blocks_c(C.byref(p), workgroups, 256) == (wide < narrow)
+
+
+@pytest.mark.parametrize("rows,columns", [(8, 9), (8, 15), (54, 73), (63, 71), (9, 100), (301, 86), (128, 17), (27, 1187), (65, 9)])
+def test_bands_hold_every_tile_once_and_few_columns_an_xcd(rules, rows, columns):
+    tiles = (C.c_uint32 * (rows * columns + 8))()
+    count = rules.dot_bands_c(rows, columns, tiles)
+    assert rows * columns <= count < rows * columns + 8
+    order = list(tiles[:count])
+    assert sorted(t for t in order if t != 0xFFFFFFFF) == sorted(65536 * r + c for r in range(rows) for c in range(columns))
+    for xcd in range(8):
+        mine = [t for t in order[xcd::8] if t != 0xFFFFFFFF]
+        assert len(mine) <= -(-rows * columns // 8)
+        assert len({t % 65536 for t in mine}) <= 2 * -(-columns // 8) + 1  # parts of two bands, at the end of three
+
+
+def test_whole_eights_of_columns_and_small_launches_keep_the_plain_grid(rules):
+    for rows, columns in ((100, 8), (100, 72), (7, 73), (300, 5), (1, 1187)):
+        assert rules.dot_bands_c(rows, columns, None) == 0

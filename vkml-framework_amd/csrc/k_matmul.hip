@@ -63,6 +63,7 @@ struct MatmulDotArgs {
     float* out;           // [M, N]
     uint32_t m, n, k;
     const float* residual;  // [M, N] added to each output, or null
+    DotBands bands;  // the order of the tiles over the grid
 };
 
 // out[row, col] = v, or residual[row, col] + v (the binary add that
@@ -427,7 +428,9 @@ __global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulD
     __shared__ StagedLds<FMT, F16S, RT, CT> l;
     const uint32_t t = thread_index(), lane = t % kWave, wave = t / kWave;
     const uint32_t g = lane / 16, li = lane % 16;
-    const uint32_t row0 = blockIdx.y * S::TM, col0 = blockIdx.x * S::TN;
+    uint32_t tile_row = blockIdx.y, tile_col = blockIdx.x;
+    if (p.bands.width != 0 && !p.bands.tile(blockIdx.x, tile_row, tile_col)) return;
+    const uint32_t row0 = tile_row * S::TM, col0 = tile_col * S::TN;
     const uint32_t blocks = p.k / 32;
     float acc[RT][CT][4];
 #pragma unroll
@@ -506,8 +509,9 @@ __global__ void __launch_bounds__(kT, RT * CT == 4 ? 4 : 1) k_matmul_dot(MatmulD
 }
 
 template <int FMT, bool F16S, int RT, int CT>
-void launch_tile(const MatmulDotArgs& p) {
-    const dim3 grid((p.n + 64 * CT - 1) / (64 * CT), (p.m + 16 * RT - 1) / (16 * RT));
+void launch_tile(MatmulDotArgs p) {
+    p.bands = dot_bands((p.m + 16 * RT - 1) / (16 * RT), (p.n + 64 * CT - 1) / (64 * CT));
+    const dim3 grid = p.bands.width != 0 ? dim3(8 * p.bands.share) : dim3(p.bands.columns, p.bands.rows);
     const auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kT), 0, vkml::abi::stream(), p); };
     const DotTail tail = dot_tail(RT, CT, p.k);
     if constexpr (RT * CT == 8) {
@@ -547,7 +551,7 @@ int matmul_dot_common(const char* what, const vkml_gemv_dot_params* p, const voi
     if (p->m == 0 || p->n == 0) return VKML_OK;
     VKML_CHECK_ARG(a_values && b_values && out && b_scales && a_scales, name + ": null buffer");
     const MatmulDotArgs args{static_cast<const uint8_t*>(a_values), a_scales, static_cast<const uint8_t*>(b_values), b_scales, out,
-                             p->m, p->n, p->k, residual};
+                             p->m, p->n, p->k, residual, {}};
     vkml::abi::ProfileScope prof(what);
     const bool f16 = p->scale_type == VKML_F16;
     switch (p->b_type) {

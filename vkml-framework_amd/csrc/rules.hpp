@@ -1,6 +1,6 @@
 // rules.hpp -- which kernel of a family a call takes, where that follows from
-// its sizes and addresses alone: host code without HIP, so that the choices
-// can be checked on any machine. What each line rests on stands beside it.
+// its sizes and addresses alone: code without HIP, so that the choices can be
+// checked on any machine. What each line rests on stands beside it.
 #pragma once
 
 #include <cstdint>
@@ -116,6 +116,45 @@ inline DotTile dot_tile(uint32_t b_type, bool f16_scales, uint32_t m, uint32_t n
     if (waves(2, 2) >= (b_type == VKML_Q8_0 && f16_scales ? 1280 : 1600)) return {2, 2};
     if (dot_has_16x128(b_type, f16_scales) && waves(2, 2) >= 900) return {1, 2};
     return {1, 1};
+}
+
+// How k_matmul_dot's rows x columns tiles lie on its grid. Workgroups go to the
+// eight XCDs in turn, each with an L2 of its own. With whole eights of column
+// tiles, a grid (columns, rows) leaves each XCD an eighth of them, whose
+// weights its row tiles find in its L2. With any other number every XCD reads
+// all of the weights, from the last-level cache: q8_0 1719 x 9223 x 6848 (73
+// columns of 32 x 128 tiles) took 790 us where 72 columns took 508. Then the
+// tiles are numbered band by band of an eighth of the columns, row by row in a
+// band, and each XCD takes a contiguous eighth of that order (width 0: the
+// plain grid): 524 us; 2000 x 9000 x 8192 884 -> 688, q4_0 1719 x 9223 x 4160
+// 361 -> 281.
+#ifdef __HIPCC__
+#define VKML_RULES_BOTH __host__ __device__
+#else
+#define VKML_RULES_BOTH
+#endif
+struct DotBands {
+    uint32_t rows, columns;
+    uint32_t width;  // columns of a band
+    uint32_t share;  // tiles of an XCD
+
+    // The tile of workgroup i of 8 share; whether it has one.
+    VKML_RULES_BOTH bool tile(uint32_t i, uint32_t& row, uint32_t& col) const {
+        const uint32_t s = i % 8 * share + i / 8;
+        if (s >= rows * columns) return false;
+        const uint32_t band = s / (width * rows), at = s % (width * rows), first = band * width;
+        const uint32_t w = columns - first < width ? columns - first : width;
+        row = at / w;
+        col = first + at % w;
+        return true;
+    }
+};
+
+// (A launch of few tiles reads little twice; rows * columns fits 32 bits.)
+inline DotBands dot_bands(uint32_t rows, uint32_t columns) {
+    const uint64_t tiles = static_cast<uint64_t>(rows) * columns;
+    const bool bands = columns % 8 != 0 && columns > 8 && rows >= 8 && tiles < (1u << 31);
+    return {rows, columns, bands ? (columns + 7) / 8 : 0, static_cast<uint32_t>((tiles + 7) / 8)};
 }
 
 // The last chunk of K, 8 blocks of 32, in k_matmul_dot: whole
