@@ -280,12 +280,13 @@ def test_matmul_dot_bit_exact(fmt, f16, m, n, k):
 
 
 @pytest.mark.parametrize("fmt,f16", [(H.Q8_0, True), (H.Q8_0, False), (H.Q4_0, True), (H.Q4_1, True), (H.Q4_1, False), (H.Q4_K, True)])
-@pytest.mark.parametrize("m,n,k", [(9, 70, 96), (33, 65, 288), (17, 1000, 2336), (150, 2500, 544), (119, 8200, 544), (139, 8200, 32),
+@pytest.mark.parametrize("m,n,k", [(9, 70, 96), (33, 65, 288), (17, 1000, 2336), (150, 2500, 544), (119, 8200, 544), (139, 8200, 32), (290, 4620, 352),
                                    (530, 3872, 800), (2050, 8200, 288)])
 def test_matmul_dot_tiles_bit_exact(fmt, f16, m, n, k):
     # The tiles of dot_tile's rule (16 x 64 in the first four; 16 x 128 with
-    # 1028 waves of 32 x 32 for q4_K and q4_1 with f32 scales; 32 x 128 with
-    # 1285 for q8_0 and 2057 for all; 64 x 128 for q4_0 and q4_K), ragged both
+    # 1028 waves of 32 x 32 for q4_K and q4_1 with f32 scales, 1285 for q4_1,
+    # 1450 for q4_0; 32 x 128 with 1285 for q8_0 and 2057 for all; 64 x 128 for
+    # q4_0 and q4_K), the last four in bands or not, ragged both
     # ways, with a K that ends inside a chunk of 8 blocks and of one, two and
     # several chunks.
     if fmt == H.Q4_K:

@@ -142,6 +142,13 @@ def test_last_chunk_of_matmul_dot(rules, rt, ct, k, masked, cut):
 
 # us of vkml_matmul_dot with tiles of 64 x 128, 32 x 128, 16 x 128 and 16 x 64 outputs (f16 scales or f32)
 DOT_TILES = [
+    (H.Q4_1, 1, 909, 1737, 4096, (None, 52.8, 71.5, 58.4)), (H.Q4_1, 1, 909, 1664, 4096, (None, 52.2, 49.2, 52.8)), (H.Q4_0, 1, 909, 1664, 4096, (None, 50.6, 47.9, 50)),
+    (H.Q4_1, 1, 1000, 1800, 1024, (None, 16.3, 20.7, 19.3)), (H.Q4_1, 0, 909, 1737, 4096, (None, 55.3, 57.2, 59.8)),
+    (H.Q4_0, 1, 160, 9216, 4096, (70.3, 50, 47.8, 49.5)),
+    (H.Q4_0, 1, 265, 5574, 1056, (20.6, 16.1, 15.6, 16.5)),
+    (H.Q4_1, 1, 160, 9216, 4096, (85.3, 52.7, 48.6, 50.8)),
+    (H.Q4_1, 1, 352, 4096, 4096, (83.6, 52.7, 48.2, 49.7)),
+    (H.Q4_1, 1, 265, 5574, 1056, (23.9, 17.3, 16.1, 18.7)),
     (H.Q4_K, 1, 16, 4096, 4096, (66.4, 38.7, 25.5, 19.7)),
     (H.Q4_K, 1, 64, 8192, 2048, (35.5, 20.8, 14.4, 13.7)),
     (H.Q4_K, 1, 128, 8192, 2048, (35.7, 21.2, 18, 19.4)),
@@ -266,7 +273,7 @@ DOT_TILES = [
 def test_matmul_dot_takes_a_tile_within_9_percent_of_the_fastest(rules, b_type, f16, m, n, k, us):
     # (two of 300 x 8192 x 2048 are past 6)
     picked = (42, 22, 12, 11).index(rules.dot_tile_c(b_type, f16, m, n))
-    assert us[picked] <= 1.09 * min(us)
+    assert us[picked] <= 1.09 * min(u for u in us if u)
 
 
 # us of vkml_attend_prompt_fast with blocks of 32 and of 64 keys: (heads, kv_heads, head_dim, first, queries)

@@ -532,7 +532,7 @@ void launch(const MatmulDotArgs& p) {
     if constexpr (dot_has_64_rows(FMT)) {
         if (tile.rt == 4) return launch_tile<FMT, F16S, 4, 2>(p);
     }
-    if constexpr (dot_has_16x128(FMT, F16S)) {
+    if constexpr (FMT != VKML_Q8_0) {
         if (tile.rt == 1 && tile.ct == 2) return launch_tile<FMT, F16S, 1, 2>(p);
     }
     tile.rt == 2 ? launch_tile<FMT, F16S, 2, 2>(p) : launch_tile<FMT, F16S, 1, 1>(p);

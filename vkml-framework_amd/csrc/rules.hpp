@@ -96,25 +96,34 @@ struct DotTile {
 // x 4096 x 4096 287, 292, 383, 469; 40 and 64 x 14336 x 4096 (896) 29.1 and
 // 36.2 in 16 x 64, 31.9 and 33.2 in 16 x 128.
 // q4_0: 256 x 4096 x 4096 (1024) 69, 43, 37, 31; 300 x 4096 x 4096 (1280) 69,
-// 50, 48, 36; 384 x 4096 x 4096 (1536) 70, 50, 48, 49; 512 x 4096 x 4096 (2048)
-// 71, 52, 57, 58.
+// 50, 48, 36; 160 x 9216 x 4096 (1440) 70, 50, 47.8, 49.5; 512 x 4096 x 4096
+// (2048) 71, 52, 57, 58.
 // q8_0: 256 x 4096 x 4096 68, 41, 36, 34; 131 x 8192 x 2048 (1280) 36, 25.4,
 // 26.9, 26.5; 128 x 14336 x 4096 72, 51, 75, 63; 4096 x 4096 x 4096 334, 307,
 // 449, 448; with f32 scales 131 x 8192 x 2048 32, 24.3, 24.3, 21.5.
-// q4_1: 4096 x 4096 x 4096 311, 299, 433, 453; with f32 scales 384 x 4096 x
+// q4_1: 352 x 4096 x 4096 (1408) 84, 52.7, 48.2, 49.7; 265 x 5574 x 1056 (1575)
+// 24, 17.3, 16.1, 18.7; 4096 x 4096 x 4096 311, 299, 433, 453; with f32 scales 384 x 4096 x
 // 4096 77, 56, 48, 53; 3000 x 6144 x 4096 422, 386, 456, 567.
 // (16 x 256 and 32 x 256 tiles lost throughout: 213 to 241 VGPRs. A second
 // chunk in flight in registers gained up to 4% at q4_K products of few
 // workgroups and lost 15 to 20% on the other formats, whose scales take more
 // registers.)
 constexpr bool dot_has_64_rows(uint32_t b_type) { return b_type == VKML_Q4_0 || b_type == VKML_Q4_K; }
-constexpr bool dot_has_16x128(uint32_t b_type, bool f16_scales) { return b_type == VKML_Q4_K || (b_type == VKML_Q4_1 && !f16_scales); }
+// From how many waves of a 32 x 32 tile on a 16 x 128 one (not q8_0).
+constexpr uint64_t dot_16x128_line(uint32_t b_type, bool f16_scales) {
+    return b_type == VKML_Q4_0 ? 1400 : b_type == VKML_Q4_1 && f16_scales ? 1280 : b_type == VKML_Q8_0 ? ~0ull : 900;
+}
 
 inline DotTile dot_tile(uint32_t b_type, bool f16_scales, uint32_t m, uint32_t n) {
     const auto waves = [&](uint64_t rt, uint64_t ct) { return ((m + 16 * rt - 1) / (16 * rt)) * ((n + 16 * ct - 1) / (16 * ct)); };
     if (dot_has_64_rows(b_type) && waves(4, 2) >= 8192) return {4, 2};
-    if (waves(2, 2) >= (b_type == VKML_Q8_0 && f16_scales ? 1280 : 1600)) return {2, 2};
-    if (dot_has_16x128(b_type, f16_scales) && waves(2, 2) >= 900) return {1, 2};
+    // (q4_0's and q4_1's 16 x 128 tile holds three workgroups a compute unit;
+    // one more round of them loses: q4_1 909 x 1737 x 4096, 798 workgroups,
+    // 52.8, 71.5 us, 909 x 1664 x 4096, 741, 52.2, 49.2)
+    const bool mid = waves(2, 2) >= dot_16x128_line(b_type, f16_scales);
+    const bool second_round = b_type != VKML_Q4_K && waves(1, 2) > 4 * 3 * 256;
+    if (waves(2, 2) >= (b_type == VKML_Q8_0 && f16_scales ? 1280 : 1600) || (mid && second_round)) return {2, 2};
+    if (mid) return {1, 2};
     return {1, 1};
 }
 
