@@ -83,6 +83,7 @@ def test_short_sums_that_end_in_a_chunks_first_half_are_cut(rules):
 
 # us of probs v (f16, heads, queries, first query's position, head_dim)
 PROBS_V_TILES = [
+    (32, 147, 0, 128, (22, 11, 8.85, 7.02)),
     (8, 1000, 0, 80, (118, 67.6, 44, 28.5)),
     (8, 2048, 2048, 128, (476, 295, 268, 251)),
     (32, 512, 0, 64, (62.5, 35.8, 23.7, 16.1)),
@@ -310,3 +311,28 @@ def test_bands_hold_every_tile_once_and_few_columns_an_xcd(rules, rows, columns)
 def test_whole_eights_of_columns_and_small_launches_keep_the_plain_grid(rules):
     for rows, columns in ((100, 8), (100, 72), (7, 73), (300, 5), (1, 1187)):
         assert rules.dot_bands_c(rows, columns, None) == 0
+
+
+# us of transposed f16 products of short sums, wave tiles as above
+SHORT_SUMS = [
+    (64, 1000, 8, (4.24, 3.75, 3.13, 3.34)),
+    (64, 1000, 64, (9.96, 6.19, 4.46, 3.34)),
+    (130, 9532, 32, (7.08, 5.82, 5.35, 8.11)),
+    (130, 9532, 72, (11.96, 10.47, 8.71, 12.06)),
+    (130, 9532, 128, (17.79, 13.44, 11.38, 12.05)),
+    (235, 12080, 12, (7.61, 6.63, 6.86, 13.83)),
+    (235, 12080, 80, (17.37, 14.54, 14.14, 20.96)),
+    (518, 5040, 16, (7.72, 6.61, 6.45, 12.93)),
+    (518, 5040, 144, (27.11, 21.93, 20.76, 26.8)),
+    (1188, 2272, 88, (18.85, 15.64, 16.38, 19.9)),
+    (1188, 2272, 192, (34.77, 26.74, 26.86, 27.19)),
+    (2008, 6992, 16, (18.67, 19.68, 19.16, 51.29)),
+    (400, 1000, 16, (5.18, 3.93, 3.3, 4.29)),
+    (400, 1000, 80, (12.18, 7.71, 5.65, 5.89)),
+]
+
+
+@pytest.mark.parametrize("m,n,k,us", SHORT_SUMS)
+def test_short_sums_take_a_tile_within_10_percent_of_the_fastest(rules, m, n, k, us):
+    picked = (42, 22, 21, 11).index(rules.wave_tile_c(C.byref(_matmul(m, n, k, H.F16, 1))))
+    assert us[picked] <= 1.1 * min(us)

@@ -56,10 +56,23 @@ inline WaveTile wave_tile(const vkml_matmul_params& p) {
     const auto waves = [&](uint64_t r, uint64_t nc) {
         return seen * static_cast<double>((p.m + 16 * nc - 1) / (16 * nc) * ((p.n + 16 * r - 1) / (16 * r)) * p.batches);
     };
-    const bool quant = p.b_type >= VKML_Q8_0;
-    if (p.b_type != VKML_Q4_K && waves(4, 2) >= 16384) return {4, 2};
-    if (waves(2, 2) >= (quant ? 3072 : 8192)) return {2, 2};
-    if (waves(2, 1) >= (quant ? 3584 : 6144)) return {2, 1};
+    if (p.b_type >= VKML_Q8_0) {
+        if (p.b_type != VKML_Q4_K && waves(4, 2) >= 16384) return {4, 2};
+        if (waves(2, 2) >= 3072) return {2, 2};
+        if (waves(2, 1) >= 3584) return {2, 1};
+        return {1, 1};
+    }
+    // The smallest tile multiplies whole chunks of 64 k's, the others chunks of
+    // 32 or parts of one: short sums that leave half of a last 64 empty go to
+    // the others from fewer waves on (f16, 130 x 9532 x 72 12.0, 10.5, 8.7, 12.1;
+    // 1188 x 2272 x 88 18.9, 15.6, 16.4, 19.9; 518 x 5040 x 16 7.7, 6.6, 6.5,
+    // 12.9, where the kernel before took 7.9).
+    // Element loads (a ragged k) and b [k, n]'s tails, which only the 32 x 64
+    // tile cuts, leave less of that.
+    const bool half = (p.k - 1) % 64 < 32, tiny = half && p.k <= 32 && p.k % 4 == 0, brief = half && p.k <= 160 && (p.b_transposed || p.k <= 32);
+    if (waves(4, 2) >= (tiny ? 4096 : 16384)) return {4, 2};
+    if (waves(2, 2) >= (tiny ? 2048 : 8192)) return {2, 2};
+    if (waves(2, 1) >= (tiny ? 512 : brief ? 1024 : 6144)) return {2, 1};
     return {1, 1};
 }
 
