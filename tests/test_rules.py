@@ -308,8 +308,9 @@ def test_bands_hold_every_tile_once_and_few_columns_an_xcd(rules, rows, columns)
         assert len({t % 65536 for t in mine}) <= 2 * -(-columns // 8) + 1  # parts of two bands, at the end of three
 
 
-def test_whole_eights_of_columns_and_small_launches_keep_the_plain_grid(rules):
-    for rows, columns in ((100, 8), (100, 72), (7, 73), (300, 5), (1, 1187)):
+def test_whole_eights_of_columns_and_small_and_huge_launches_keep_the_plain_grid(rules):
+    # (the huge ones: 256 work items a tile along x would pass 32 bits)
+    for rows, columns in ((100, 8), (100, 72), (7, 73), (300, 5), (1, 1187), (31250, 1187), (65535, 129)):
         assert rules.dot_bands_c(rows, columns, None) == 0
 
 

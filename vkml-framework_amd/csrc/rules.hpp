@@ -172,10 +172,11 @@ struct DotBands {
     }
 };
 
-// (A launch of few tiles reads little twice; rows * columns fits 32 bits.)
+// (A launch of few tiles reads little twice; a grid's work items along x, 256
+// a tile, fit 32 bits.)
 inline DotBands dot_bands(uint32_t rows, uint32_t columns) {
     const uint64_t tiles = static_cast<uint64_t>(rows) * columns;
-    const bool bands = columns % 8 != 0 && columns > 8 && rows >= 8 && tiles < (1u << 31);
+    const bool bands = columns % 8 != 0 && columns > 8 && rows >= 8 && tiles < (1u << 23);
     return {rows, columns, bands ? (columns + 7) / 8 : 0, static_cast<uint32_t>((tiles + 7) / 8)};
 }
 
